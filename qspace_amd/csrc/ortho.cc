@@ -249,14 +249,19 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   hipStream_t s = default_stream();
   std::vector<SvdGather> gath;
   std::vector<SvdItem> items;
-  int64_t work = 0, nsig = 0;
+  std::vector<SvdGroup> qr;  // the groups reduced by QR; the others in `big`
+  std::vector<int32_t> big;
+  int64_t work = 0, nsig = 0, nperm = 0;
+  auto take = [&](int64_t n) {  // buffers start at multiples of 16 doubles
+    const int64_t o = work;
+    work += (n + 15) & ~(int64_t)15;
+    return o;
+  };
   for (auto& b : G) {
     if (b.n == 0) continue;
     if (b.n > INT32_MAX || b.m > INT32_MAX) fail(QSX_ERR_UNSUPPORTED, "orthoQS: group matrix too large");
-    b.a_off = work;
-    work += b.m * b.n;
-    b.v_off = work;
-    work += b.n * b.n;
+    b.a_off = take(b.m * b.n);
+    b.v_off = take(b.n * b.n);
     b.s_off = nsig;
     nsig += b.n;
     b.item = (int)items.size();
@@ -266,7 +271,25 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
     it.s_off = b.s_off;
     it.m = (int32_t)b.m;
     it.n = (int32_t)b.n;
-    it.lds = (b.m * b.n + b.n * b.n) <= SVD_LDS_DOUBLES ? 1 : 0;
+    if (b.m <= SVD_QR_MAX_M && b.n <= SVD_QR_MAX_N) {
+      SvdGroup q{};
+      q.a = b.a_off;
+      q.v = b.v_off;
+      q.s = b.s_off;
+      q.m = it.m;
+      q.n = it.n;
+      q.ldf = (it.m + 15) & ~15;
+      q.n16 = (it.n + 15) & ~15;
+      q.perm = (int32_t)nperm;
+      nperm += it.n;
+      q.x = take((int64_t)it.n * it.n);
+      q.w = take((int64_t)it.n * it.n);
+      q.c1 = take((int64_t)q.ldf * q.n16);
+      q.c2 = take((int64_t)q.n16 * q.n16);
+      qr.push_back(q);
+    } else {
+      big.push_back((int32_t)items.size());
+    }
     items.push_back(it);
     for (size_t t = 0; t < b.blk.size(); ++t) {
       const int i = b.blk[t];
@@ -297,11 +320,78 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
     }
   }
   if (nsig == 0) fail(QSX_ERR_ARG, "orthoQS: got empty SVD data");
+  // the QR factorisations (all groups', then the second ones), the groups
+  // decomposed in LDS (one workgroup each) and in rounds of column blocks,
+  // and the tiles the reflectors are applied to
+  std::vector<SvdQr> qr1, qr2;
+  std::vector<SvdApply> app;
+  std::vector<SvdItem> unit;           // W = I of the groups in rounds
+  std::vector<int32_t> small, unitidx;
+  std::vector<SvdBlockStep> rsteps;    // one sweep: the rounds back to back
+  std::vector<size_t> roff(1, 0);
+  int maxrows = 0, maxn = 0, maxnb = 0;
+  std::vector<int32_t> mid, nbr, cbr;
+  for (size_t i = 0; i < qr.size(); ++i) {
+    const SvdGroup& q = qr[i];
+    const int64_t nt = (int64_t)(q.n16 / 16) * 256;
+    SvdQr a{q.a, take((int64_t)q.ldf * q.n16), take(nt), q.x, q.m, q.n, q.ldf, q.perm, (int32_t)i, 0};
+    qr1.push_back(a);
+    for (int c = 0; c < q.n; c += 64) app.push_back({a.f, a.t, q.c1, q.a, q.m, q.n, q.ldf, -1, c, 0});
+    SvdQr b{q.x, take((int64_t)q.n16 * q.n16), take(nt), q.x, q.n, q.n, q.n16, -1, (int32_t)i, 0};
+    qr2.push_back(b);
+    for (int c = 0; c < q.n; c += 64) app.push_back({b.f, b.t, q.c2, q.v, q.n, q.n, q.n16, q.perm, c, 0});
+    maxrows = std::max(maxrows, q.ldf);
+    maxn = std::max(maxn, q.n);
+    if (q.n <= SVD_LDS_N) {
+      small.push_back((int32_t)i);
+      continue;
+    }
+    // an even number of blocks of an even number of columns, at most SVD_CROSS_COLS
+    const int nb = 2 * ((q.n + 2 * SVD_CROSS_COLS - 1) / (2 * SVD_CROSS_COLS));
+    const int cb = ((q.n + nb - 1) / nb + 1) & ~1;
+    mid.push_back((int32_t)i);
+    nbr.push_back(nb);
+    cbr.push_back(cb);
+    maxnb = std::max(maxnb, nb);
+    SvdItem u{};
+    u.v_off = q.w;
+    u.m = u.n = q.n;
+    unitidx.push_back((int32_t)unit.size());
+    unit.push_back(u);
+  }
+  // a sweep: the pairs within every column block, then the pairs across
+  // blocks P, Q in the round-robin order of the blocks
+  for (int st = -1; st < maxnb - 1; ++st) {
+    for (size_t a = 0; a < mid.size(); ++a) {
+      const int nb = nbr[a], cb = cbr[a], n = qr[mid[a]].n;
+      if (st >= nb - 1) continue;
+      for (int k = 0; k < (st < 0 ? nb : nb / 2); ++k) {
+        SvdBlockStep b{};
+        b.grp = mid[a];
+        const int P0 = st < 0 ? k : k == 0 ? nb - 1 : (st + k) % (nb - 1);
+        b.p0 = std::min(n, P0 * cb);
+        b.p1 = std::min(n, (P0 + 1) * cb);
+        if (st < 0) {
+          b.q0 = b.q1 = b.p1;
+          if (b.p1 - b.p0 < 2) continue;
+        } else {
+          const int Q0 = k == 0 ? st : (st - k + nb - 1) % (nb - 1);
+          b.q0 = std::min(n, Q0 * cb);
+          b.q1 = std::min(n, (Q0 + 1) * cb);
+          if (b.p1 == b.p0 || b.q1 == b.q0) continue;
+        }
+        if (b.p1 - b.p0 > SVD_CROSS_COLS || b.q1 - b.q0 > SVD_CROSS_COLS)
+          fail(QSX_ERR_STRUCT, "orthoQS: internal column block too large");
+        rsteps.push_back(b);
+      }
+    }
+    roff.push_back(rsteps.size());
+  }
   // every access of the kernels inside its buffer (checked before launch)
   for (const SvdItem& it : items) {
     const int64_t mn = (int64_t)it.m * it.n, nn = (int64_t)it.n * it.n;
     if (it.m < it.n || it.n < 1 || it.a_off < 0 || it.a_off + mn > work || it.v_off + nn > work ||
-        it.s_off + it.n > nsig || (it.lds && mn + nn > SVD_LDS_DOUBLES))
+        it.s_off + it.n > nsig)
       fail(QSX_ERR_STRUCT, "orthoQS: internal SVD item out of range");
   }
   for (const SvdGather& g : gath) {
@@ -322,16 +412,11 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
       for (void* x : p) dev_free(x);
     }
   } fr;
-  // groups that fit in LDS: one workgroup each (k_jacobi_svd); the others:
-  // block one-sided Jacobi over column blocks of at most cb columns, two
-  // blocks (and their columns of V) staged in LDS per workgroup
-  std::vector<SvdItem> small;
-  std::vector<int32_t> big, nbk, cbk;
-  for (size_t i = 0; i < items.size(); ++i) {
-    if (items[i].lds) {  // checked above: fits in LDS
-      small.push_back(items[i]);
-      continue;
-    }
+  // groups beyond the QR's range: block one-sided Jacobi over column blocks
+  // of at most cb columns, two blocks (and their columns of V) staged in LDS
+  // per workgroup
+  std::vector<int32_t> nbk, cbk;
+  for (int32_t i : big) {
     const int64_t m = items[i].m, n = items[i].n;
     const int64_t cmax = SVD_LDS_DOUBLES / (2 * (m + n));
     if (cmax < 1) fail(QSX_ERR_UNSUPPORTED, "orthoQS: group matrix %lld x %lld too large", (long long)m, (long long)n);
@@ -340,27 +425,39 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
     if (nb < 2) nb = 2;
     const int64_t cb = (n + nb - 1) / nb;
     if (2 * cb * (m + n) > SVD_LDS_DOUBLES) fail(QSX_ERR_STRUCT, "orthoQS: internal column block too large");
-    big.push_back((int32_t)i);
     nbk.push_back((int32_t)nb);
     cbk.push_back((int32_t)cb);
   }
+  std::vector<UploadPart> up;
+  auto put = [&](auto& v) {
+    using T = typename std::decay_t<decltype(v)>::value_type;
+    T* d = (T*)fr.add(sizeof(T) * std::max<size_t>(1, v.size()));
+    if (!v.empty()) up.push_back({d, v.data(), sizeof(T) * v.size()});
+    return d;
+  };
+  SvdItem* ditems = put(items);
+  SvdGather* dgath = put(gath);
+  int32_t* dbig = put(big);
+  SvdGroup* dqr = put(qr);
+  SvdQr* dqr1 = put(qr1);
+  SvdQr* dqr2 = put(qr2);
+  SvdApply* dapp = put(app);
+  SvdItem* dunit = put(unit);
+  int32_t* dunitidx = put(unitidx);
+  int32_t* dsmall = put(small);
+  SvdBlockStep* drsteps = put(rsteps);
+  int32_t* dperm = (int32_t*)fr.add(sizeof(int32_t) * std::max<int64_t>(1, nperm));
+  int32_t* dexpo = (int32_t*)fr.add(sizeof(int32_t) * std::max<size_t>(1, qr.size()));
   int32_t* dsw = (int32_t*)fr.add(sizeof(int32_t) * std::max<size_t>(1, small.size()));
-  SvdItem* dsmall = (SvdItem*)fr.add(sizeof(SvdItem) * std::max<size_t>(1, small.size()));
-  SvdItem* ditems = (SvdItem*)fr.add(sizeof(SvdItem) * items.size());
-  SvdGather* dgath = (SvdGather*)fr.add(sizeof(SvdGather) * std::max<size_t>(1, gath.size()));
-  int32_t* drot = (int32_t*)fr.add(sizeof(int32_t) * items.size());
-  int32_t* dbig = (int32_t*)fr.add(sizeof(int32_t) * std::max<size_t>(1, big.size()));
+  const size_t nrot = (size_t)jacobi_max_sweeps() * qr.size();
+  int32_t* drot = (int32_t*)fr.add(sizeof(int32_t) * std::max(nrot, items.size()));
   upload_packed(P, P.hdata, dpsi.p, s);
-  QSX_HIP(hipMemcpyAsync(ditems, items.data(), sizeof(SvdItem) * items.size(), hipMemcpyHostToDevice, s));
-  if (!small.empty())
-    QSX_HIP(hipMemcpyAsync(dsmall, small.data(), sizeof(SvdItem) * small.size(), hipMemcpyHostToDevice, s));
-  if (!big.empty())
-    QSX_HIP(hipMemcpyAsync(dbig, big.data(), sizeof(int32_t) * big.size(), hipMemcpyHostToDevice, s));
-  if (!gath.empty())
-    QSX_HIP(hipMemcpyAsync(dgath, gath.data(), sizeof(SvdGather) * gath.size(), hipMemcpyHostToDevice, s));
+  upload_many(up, s);
   Timer tm(s);
   launch_fill_zero(dwork.p, work, s);
   launch_svd_gather(dgath, (int)gath.size(), dpsi.p, dwork.p, s);
+  launch_svd_qr(dqr1, (int)qr1.size(), maxrows, dwork.p, dperm, dexpo, s);
+  launch_svd_qr(dqr2, (int)qr2.size(), SVD_QR_MAX_N, dwork.p, dperm, dexpo, s);
   // the groups in LDS run on the side stream, beside the block steps
   hipStream_t s2 = side_stream();
   struct Ev {
@@ -379,7 +476,7 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   } drain{s, s2};
   QSX_HIP(hipEventRecord(ready.e, s));
   QSX_HIP(hipStreamWaitEvent(s2, ready.e, 0));
-  launch_jacobi_svd(dsmall, (int)small.size(), dwork.p, dsig.p, dsw, s2);
+  launch_jacobi_lds(dqr, dsmall, (int)small.size(), dwork.p, dsw, s2);
   QSX_HIP(hipEventRecord(done.e, s2));
   int maxsw = 0;
   if (!big.empty()) {
@@ -449,7 +546,33 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
     maxsw = sw;
     launch_svd_finalize(ditems, dbig, (int)big.size(), dwork.p, dsig.p, s);
   }
+  if (!mid.empty()) {
+    launch_svd_init_v(dunit, dunitidx, (int)unit.size(), dwork.p, s);
+    QSX_HIP(hipMemsetAsync(drot, 0, sizeof(int32_t) * nrot, s));
+    // sweeps are enqueued ahead (a converged group's workgroups return at
+    // once): preconditioned matrices take 6 to 10 sweeps
+    std::vector<int32_t> rot(nrot);
+    int sw = 0;
+    bool more = true;
+    for (int ahead = 8; more && sw < jacobi_max_sweeps(); ahead = 2) {
+      for (int e = std::min(jacobi_max_sweeps(), sw + ahead); sw < e; ++sw)
+        for (size_t st = 0; st + 1 < roff.size(); ++st)
+          launch_jacobi_cross(dqr, (int)qr.size(), drsteps + roff[st], (int)(roff[st + 1] - roff[st]), dwork.p, drot,
+                              sw, s);
+      const size_t o = (size_t)(sw - 1) * qr.size();
+      QSX_HIP(hipMemcpyAsync(rot.data(), drot, sizeof(int32_t) * (o + qr.size()), hipMemcpyDeviceToHost, s));
+      QSX_HIP(hipStreamSynchronize(s));
+      more = false;
+      for (int32_t i : mid) more |= rot[o + i] != 0;
+    }
+    if (more) fail(QSX_ERR_ARG, "orthoQS: block Jacobi SVD did not converge in %d sweeps", sw);
+    for (int k = 0; k < sw; ++k)
+      for (int32_t i : mid)
+        if (rot[(size_t)k * qr.size() + i]) maxsw = std::max(maxsw, k + 2);
+  }
   QSX_HIP(hipStreamWaitEvent(s, done.e, 0));
+  launch_svd_vectors(dqr, (int)qr.size(), maxn, dwork.p, dsig.p, dexpo, s);
+  launch_svd_applyq(dapp, (int)app.size(), maxrows, dwork.p, dperm, s);
   std::vector<double> sig(nsig);
   std::vector<int32_t> sweeps(small.size());
   QSX_HIP(hipMemcpyAsync(sig.data(), dsig.p, sizeof(double) * nsig, hipMemcpyDeviceToHost, s));

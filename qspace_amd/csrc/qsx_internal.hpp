@@ -394,11 +394,17 @@ void launch_block_zero_flags(const int64_t* doffs, int nblk, const double* data,
 void launch_fill_zero(double* p, int64_t n, hipStream_t s);
 
 // ---------------------------------------------------------------- block SVD
-// (svd.hip) group matrices of the truncation, one-sided Jacobi SVD, result
-// blocks.  A group matrix is stored m x n column-major with m >= n (the
-// transpose of a wide matrix); it is decomposed by one workgroup in LDS
-// when m*n + n*n <= SVD_LDS_DOUBLES (k_jacobi_svd takes only such items),
-// by column-block steps otherwise.
+// (svd.hip, svdqr.hip) group matrices of the truncation, one-sided Jacobi SVD,
+// result blocks.  A group matrix is stored m x n column-major with m >= n
+// (the transpose of a wide matrix).  Up to SVD_QR_MAX_M x SVD_QR_MAX_N it is
+// reduced to an n x n triangle by QR first and decomposed there, in one
+// workgroup's LDS for n <= SVD_LDS_N and by rounds of column blocks beyond;
+// a larger one is decomposed as it is by column-block steps with
+// SVD_LDS_DOUBLES of LDS.
+constexpr int SVD_QR_MAX_M = 1024;
+constexpr int SVD_QR_MAX_N = 256;
+constexpr int SVD_LDS_N = 96;         // 2 n (n + 8) doubles fit a workgroup's LDS
+constexpr int SVD_CROSS_COLS = 16;    // columns per block of the cross rounds
 constexpr int SVD_LDS_DOUBLES = 20224;
 // block -> its place in a group matrix (transposed for a wide group)
 struct SvdGather {
@@ -410,7 +416,29 @@ struct SvdGather {
 // (unsorted) at s_off; on return A holds the left vectors
 struct SvdItem {
   int64_t a_off, v_off, s_off;
-  int32_t m, n, lds, pad;
+  int32_t m, n;
+};
+// a group matrix reduced by QR: results (left vectors m x n at a, right
+// vectors n x n at v, singular values at s) and the work buffers: X, W (n x n),
+// C1 (ldf x n16: U, then the left vectors), C2 (n16 x n16: W, then the right
+// vectors before the column order is undone)
+struct SvdGroup {
+  int64_t a, v, s, x, w, c1, c2;
+  int32_t m, n, ldf, n16;  // ldf, n16: m, n rounded up to 16
+  int32_t perm, pad;       // offset of the column order in the permutation array
+};
+// QR of src (m x n, leading dim m) into F (ldf x n16, zeroed by the caller),
+// T (n16/16 triangular factors of 16 x 16) and X = R^T; perm >= 0: columns in
+// order of falling norm, scaled by the power of two expo[grp]
+struct SvdQr {
+  int64_t src, f, t, x;
+  int32_t m, n, ldf, perm, grp, pad;
+};
+// columns col0 .. col0+63 of Q C (C: ldf x n16), rows 0 .. m-1 to dst (leading
+// dim m; row i to perm[i] if perm >= 0)
+struct SvdApply {
+  int64_t f, t, c, dst;
+  int32_t m, n, ldf, perm, col0, pad;
 };
 struct SvdCol {
   int32_t col, pad;
@@ -424,17 +452,28 @@ struct SvdScatter {
   double scale;  // block factor on top of the column scales
 };
 void launch_svd_gather(const SvdGather* ditems, int nitems, const double* src, double* work, hipStream_t s);
+void launch_svd_qr(const SvdQr* ditems, int nitems, int maxrows, double* work, int32_t* perm, int32_t* expo,
+                   hipStream_t s);
+void launch_svd_vectors(const SvdGroup* dgroups, int ngroups, int maxn, double* work, double* sig,
+                        const int32_t* expo, hipStream_t s);
+void launch_svd_applyq(const SvdApply* ditems, int nitems, int maxrows, double* work, const int32_t* perm,
+                       hipStream_t s);
 // sweeps[i] = sweeps that rotated (jacobi_max_sweeps(): not converged)
-void launch_jacobi_svd(const SvdItem* ditems, int nitems, double* work, double* sig, int32_t* sweeps, hipStream_t s);
+void launch_jacobi_lds(const SvdGroup* dgroups, const int32_t* dwhich, int n, double* work, int32_t* sweeps,
+                       hipStream_t s);
 int jacobi_max_sweeps();
 void launch_svd_scatter(const SvdScatter* ditems, int nitems, const SvdCol* dcols, const double* work, double* out,
                         hipStream_t s);
-// block one-sided Jacobi of group matrices beyond the LDS: one step = the
-// column-block pairs (P, Q) of a round-robin over a group's column blocks,
-// one workgroup each; rot[grp] set when a pair rotated
+// block one-sided Jacobi: one step = the column-block pairs (P, Q) of a
+// round-robin over a group's column blocks, one workgroup each (q0 == q1: the
+// pairs within P).  launch_jacobi_cross: rot[sweep * ngroups + grp] set when a
+// pair rotated (zeroed by the caller), groups done in the sweep before are
+// skipped; launch_jacobi_block: rot[grp]
 struct SvdBlockStep {
   int32_t grp, p0, p1, q0, q1, pad;
 };
+void launch_jacobi_cross(const SvdGroup* dgroups, int ngroups, const SvdBlockStep* dsteps, int nsteps, double* work,
+                         int32_t* rot, int sweep, hipStream_t s);
 void launch_jacobi_block(const SvdItem* dgroups, const SvdBlockStep* dsteps, int nsteps, double* work, int32_t* rot,
                          int sweep, hipStream_t s);
 void launch_svd_finalize(const SvdItem* dgroups, const int32_t* dwhich, int n, double* work, double* sig,

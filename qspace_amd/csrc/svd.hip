@@ -1,24 +1,32 @@
 // svd.hip -- the block SVD of the truncation (orthoQS): the group
 // matrices are assembled from the blocks on the device, each is decomposed
-// by a one-sided Jacobi SVD in one workgroup, and the kept singular vectors
-// are scattered into the blocks of the two result tensors.
+// by a one-sided Jacobi SVD, and the kept singular vectors are scattered
+// into the blocks of the two result tensors.
 //
 // One-sided Jacobi (Hestenes, J. SIAM 6 (1958); the rotation and stopping
 // rule of Demmel and Veselic, SIAM J. Matrix Anal. Appl. 13 (1992)): the
-// columns of an m x n matrix (m >= n) are orthogonalised by plane rotations
-// of column pairs; a sweep visits every pair once in the round-robin order,
-// whose n/2 pairs per step are disjoint and run in parallel.  At the end
-// a_j = sigma_j u_j and the accumulated rotations are V.
+// columns of a matrix are orthogonalised by plane rotations of column
+// pairs; a sweep visits every pair once, in steps of disjoint pairs that run
+// in parallel.  At the end x_j = sigma_j u_j and the accumulated rotations
+// are W.  Matrices of up to SVD_QR_MAX_M x SVD_QR_MAX_N are reduced to an
+// n x n triangle first (svdqr.hip); k_jacobi_lds runs all sweeps of one with
+// n <= SVD_LDS_N in a workgroup's LDS, k_jacobi_cross one round of column
+// blocks of a larger one.  Still larger matrices take k_jacobi_block, on the
+// m x n matrix itself.
 #include <cfloat>
 
 #include "qsx_internal.hpp"
+#include "svd_dev.hpp"
 
 namespace qsx {
 namespace {
 
-constexpr int SVD_NT = 1024;          // threads per workgroup
+constexpr int SVD_NT = 1024;          // threads per workgroup of k_svd_finalize
+constexpr int SVD_NT_LDS = 512;       // threads per workgroup of k_jacobi_lds
+constexpr int SVD_NT_CROSS = 256;     // threads per workgroup of k_jacobi_cross
 constexpr int SVD_NT_BLOCK = 512;     // threads per workgroup of the block steps
 constexpr int SVD_SEG = 16;           // lanes per column pair
+constexpr int SVD_SEG_CROSS = 32;     // lanes per block of columns in k_jacobi_cross
 constexpr int SVD_MAX_SWEEPS = 60;
 // Orthogonality target of a column pair: sqrt(m) eps (as LAPACK's dgesvj)
 // for the first kTightSweeps sweeps, then m eps, the rounding bound of the
@@ -28,28 +36,6 @@ constexpr int SVD_MAX_SWEEPS = 60;
 constexpr int kTightSweeps = 20;
 __host__ __device__ inline double jacobi_tol(int m, int sweep) {
   return (sweep < kTightSweeps ? sqrt((double)m) : (double)m) * DBL_EPSILON;
-}
-
-// v + (v of the lane that the DPP row pattern CTRL names); a segment is one
-// DPP row of 16 lanes, active or inactive as a whole
-template <int CTRL>
-__device__ __forceinline__ double dpp_add(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, false);
-  return v + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// sum over the 16 lanes of a segment, the same bits in every lane: pairs
-// (quad_perm 1,0,3,2), quads (quad_perm 2,3,0,1), half rows (row_half_mirror),
-// rows (row_mirror); each step adds two equal-bit partial sums in either
-// order, so all lanes agree
-__device__ __forceinline__ double seg_sum(double v) {
-  v = dpp_add<0xB1>(v);
-  v = dpp_add<0x4E>(v);
-  v = dpp_add<0x141>(v);
-  v = dpp_add<0x140>(v);
-  return v;
 }
 
 // the rotation of the Gram matrix [al ga; ga be] that zeroes ga (smaller
@@ -228,163 +214,445 @@ __device__ __forceinline__ bool jacobi_pairs(double* A, double* V, int np, int n
   return any;
 }
 
-// the cross pairs with each segment's own column of P held in registers for
-// the whole schedule: segment k owns column k of P (A and V) and meets the
-// columns of Q one step at a time, so only Q's columns move through LDS
-// (half the LDS traffic of jacobi_pairs).  m, n <= 16 R.
-template <int NT, int R>
-__device__ __forceinline__ bool jacobi_cross_reg(double* A, double* V, int np, int nq, int m, int n, double tol,
-                                                 int* flag) {
-  constexpr int L = SVD_SEG;
-  static_assert(R > 0, "register form");
-  const int tid = threadIdx.x;
-  const int seg = tid / L, lane = tid % L;
-  const int cmax = np > nq ? np : nq;
-  if (tid == 0) *flag = 0;
-  __syncthreads();
-  // one pass of segments over P's columns (np <= NT / 16, the caller's check)
-  const int k = seg;
-  const bool own = k < np;
-  double x[R], u[R];
-  double* ap = A + (int64_t)k * m;
-  double* vp = V + (int64_t)k * n;
+// the variant for column length m (longer than SVD_QR_MAX_N, or of more rows
+// than SVD_QR_MAX_M)
+template <int NT, bool CROSS>
+__device__ __forceinline__ bool jacobi_pairs_m(double* A, double* V, int np, int nq, int m, int n, double tol,
+                                               int* flag) {
+  if (m <= 512) return jacobi_pairs<NT, 32, CROSS>(A, V, np, nq, m, n, tol, flag);
+  return jacobi_pairs<NT, 0, CROSS>(A, V, np, nq, m, n, tol, flag);
+}
+
+constexpr int kColSplit = 16;  // one-wave workgroups a block's columns are dealt to (gather, scatter)
+
+// zero-padded group matrices: block e (d1 x d2, column-major) goes to
+// row i0, column j0 of its matrix (leading dim ld), transposed when trans
+__global__ __launch_bounds__(64) void k_svd_gather(const SvdGather* __restrict__ items, const double* __restrict__ src,
+                                                    double* __restrict__ work) {
+  const SvdGather it = items[blockIdx.x];
+  for (int j = blockIdx.y; j < it.d2; j += gridDim.y)
+    for (int i = threadIdx.x; i < it.d1; i += 64) {
+      const int64_t d = it.trans ? it.dst_off + j + (int64_t)i * it.ld : it.dst_off + i + (int64_t)j * it.ld;
+      work[d] = src[it.src_off + (int64_t)j * it.d1 + i] * it.scale;
+    }
+}
+
+// ---------------------------------------------------------------- n x n Jacobi
+// A segment of L = 16 or 32 lanes rotates the columns of one 2-column block P against
+// those of another, Q: the pairs (P0,Q0), (P1,Q1), then (P0,Q1), (P1,Q0),
+// with all four columns of X and of W in registers (R elements per lane and
+// column).  Two independent pairs per step share one chain of scalar work:
+// after the first level of the dot products' reduction even lanes carry the
+// first pair and odd lanes the second, so the rotation angles of both come
+// out of one instruction stream and go back to the row by DPP broadcasts.
+// The columns' squared norms are kept beside them and follow a rotation by
+// |x|^2 -/+ t ga; they are summed anew when a rotation cancels most of one,
+// and at the start of every sweep.
+//
+// Bound: the dependent chain of a step (dot, reduction, angle, update,
+// barrier).  Against one pair per segment with both columns and all three
+// sums through LDS, and the angle from three divisions and three square
+// roots (1.7 us a step at n = 64, m = 128): 0.8 us a step at n = 64.  17
+// groups of an SU(2) MPS tensor (up to 128 x 64): 2.1 ms in 20 sweeps, now
+// 0.37 ms in 7 on their R2^T.  Measured no faster: 32 lanes a segment in LDS
+// (0.47 against 0.43 ms), W's rotation beside the next angles (0.55 ms).
+template <int R>
+struct Cols2 {
+  double x[2][R], w[2][R], nn[2];
+};
+
+// The rotation of the Gram matrix [al ga; ga be] that zeroes ga (smaller
+// angle): x' = c x - s y, y' = s x + c y; with h^2 = (be-al)^2 + 4 ga^2,
+// cos 2t = |be-al| / h, c^2 = (1 + cos 2t) / 2, s = ga / (h c).  The three
+// are scaled by the larger norm's power of two first, so no square leaves the
+// range.  No rotation (c = 1, s = 0) when |ga| <= tol sqrt(al be), or when a
+// column is below tol times the other (norms): such a column is rounding
+// noise of a rank-deficient matrix (its singular value is below what FP64
+// resolves against the larger one), and rotating it against the larger
+// column only makes new noise of the same size.  al, be become the new
+// squared norms; cancel: one of them lost most of its digits.
+__device__ __forceinline__ bool jacobi_angle(double& al, double& be, double ga, double tol2, double& c, double& s,
+                                             bool& cancel) {
+  const int e = __builtin_amdgcn_frexp_exp(fmax(al, be));
+  const double a = ldexp(al, -e), b = ldexp(be, -e), g = ldexp(ga, -e);
+  const bool rot = g * g > tol2 * a * b && fmin(a, b) > tol2 * fmax(a, b);
+  const double d = b - a;
+  const double r = rsqrt_d(fma(d, d, 4.0 * g * g));
+  const double q = fma(0.5 * fabs(d), r, 0.5);
+  const double rc = rsqrt_d(q);
+  const double sn = (d >= 0.0 ? g : -g) * r * rc;
+  const double t = sn * rc;
+  const double an = fmax(fma(-t, g, a), 0.0), bn = fmax(fma(t, g, b), 0.0);
+  c = rot ? q * rc : 1.0;
+  s = rot ? sn : 0.0;
+  cancel = rot && (an < 0x1p-10 * a || bn < 0x1p-10 * b);
+  al = rot ? ldexp(an, e) : al;
+  be = rot ? ldexp(bn, e) : be;
+  return rot;
+}
+
+// the other half's value added, for segments of two rows (L = 32)
+template <int L>
+__device__ __forceinline__ double add_row(double v) {
+  if constexpr (L == 16) return v;
+  else return row_pair_sum(v);
+}
+
+template <int L, int R>
+__device__ __forceinline__ double norm2(const double (&x)[R]) {
+  double s = 0.0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) s += x[r] * x[r];
+  return add_row<L>(seg_sum(s));
+}
+
+template <int R>
+__device__ __forceinline__ void rotate_cols(double (&x)[R], double (&y)[R], double c, double s) {
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const int i = lane + L * r;
-    x[r] = own && i < m ? ap[i] : 0.0;
-    u[r] = own && i < n ? vp[i] : 0.0;
+    const double a = x[r], b = y[r];
+    x[r] = c * a - s * b;
+    y[r] = s * a + c * b;
   }
-  for (int step = 0; step < cmax; ++step) {
-    const int j = (k + step) % cmax;
-    if (own && j < nq) {
-      double* aq = A + (int64_t)(np + j) * m;
-      double* vq = V + (int64_t)(np + j) * n;
-      double y[R], z[R];
+}
+
+// the pairs (P0, Q[CR]) and (P1, Q[1-CR]); true (for the wave's active
+// segments) if any of them rotated
+template <int L, int R, int CR>
+__device__ __forceinline__ bool rotate_pairs(Cols2<R>& P, Cols2<R>& Q, double tol2, int lane) {
+  double g0 = 0.0, g1 = 0.0;
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int i = lane + L * r;
-        y[r] = i < m ? aq[i] : 0.0;
+  for (int r = 0; r < R; ++r) {
+    g0 += P.x[0][r] * Q.x[CR][r];
+    g1 += P.x[1][r] * Q.x[1 - CR][r];
+  }
+  const bool odd = lane & 1;
+  double ga = odd ? g1 : g0;
+  ga += dpp_mov<DPP_XOR1>(odd ? g0 : g1);
+  ga += dpp_mov<DPP_XOR2>(ga);
+  ga += dpp_mov<DPP_ROR4>(ga);
+  ga += dpp_mov<DPP_ROR8>(ga);
+  ga = add_row<L>(ga);
+  double al = odd ? P.nn[1] : P.nn[0], be = odd ? Q.nn[1 - CR] : Q.nn[CR];
+  double c, s;
+  bool cancel;
+  const bool rot = jacobi_angle(al, be, ga, tol2, c, s, cancel);
+  // a row's lanes may differ in the last bit of ga: its lanes 0 and 1 decide
+  // (both rows of a segment hold the same sums there)
+  if (!__any(rot && (lane & 15) < 2)) return false;
+  const double c0 = dpp_mov<DPP_BCAST<0>>(c), s0 = dpp_mov<DPP_BCAST<0>>(s);
+  const double c1 = dpp_mov<DPP_BCAST<1>>(c), s1 = dpp_mov<DPP_BCAST<1>>(s);
+  P.nn[0] = dpp_mov<DPP_BCAST<0>>(al);
+  P.nn[1] = dpp_mov<DPP_BCAST<1>>(al);
+  Q.nn[CR] = dpp_mov<DPP_BCAST<0>>(be);
+  Q.nn[1 - CR] = dpp_mov<DPP_BCAST<1>>(be);
+  rotate_cols(P.x[0], Q.x[CR], c0, s0);
+  rotate_cols(P.x[1], Q.x[1 - CR], c1, s1);
+  rotate_cols(P.w[0], Q.w[CR], c0, s0);
+  rotate_cols(P.w[1], Q.w[1 - CR], c1, s1);
+  if (__any(cancel && (lane & 15) < 2)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      P.nn[h] = norm2<L>(P.x[h]);
+      Q.nn[h] = norm2<L>(Q.x[h]);
+    }
+  }
+  return true;
+}
+
+// all pairs of P and Q
+template <int L, int R>
+__device__ __forceinline__ bool rotate_blocks(Cols2<R>& P, Cols2<R>& Q, double tol2, int lane) {
+  bool any = rotate_pairs<L, R, 0>(P, Q, tol2, lane);
+  any |= rotate_pairs<L, R, 1>(P, Q, tol2, lane);
+  return any;
+}
+
+// columns c0, c0+1 of nc columns of n rows (L (R-2) < n <= L R); an absent
+// second column is zero
+template <int L, int R>
+__device__ __forceinline__ void load_cols(Cols2<R>& b, const double* X, const double* W, int c0, int nc, int n,
+                                          int ld, int lane) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const bool ok = c0 + h < nc;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = lane + L * r;
+      const bool in = ok && (r < R - 2 || i < n);
+      b.x[h][r] = in ? X[(c0 + h) * ld + i] : 0.0;
+      b.w[h][r] = in ? W[(c0 + h) * ld + i] : 0.0;
+    }
+  }
+}
+
+template <int L, int R>
+__device__ __forceinline__ void store_cols(const Cols2<R>& b, double* X, double* W, int c0, int nc, int n, int ld,
+                                           int lane) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (c0 + h >= nc) continue;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = lane + L * r;
+      if (r < R - 2 || i < n) {
+        X[(c0 + h) * ld + i] = b.x[h][r];
+        W[(c0 + h) * ld + i] = b.w[h][r];
       }
-      double al = 0.0, be = 0.0, ga = 0.0;
+    }
+  }
+}
+
+// one sweep over all pairs of the nc columns in LDS (X, W: n rows each; nn:
+// the columns' squared norms), NT threads: the pairs within the 2-column
+// blocks (which also sums the norms), then blocks against blocks by halving:
+// at depth d each of 2^d ranges of blocks is split into P and Q, every
+// segment keeps one P block in registers and meets the Q blocks of its range
+// one round at a time.  ceil(B/2) + ceil(B/4) + ... rounds of two steps, B
+// blocks.  True (in every thread) if any pair rotated.
+template <int NT, int L, int R>
+__device__ __forceinline__ bool sweep_lds(double* X, double* W, double* nn, int nc, int n, int ld, double tol,
+                                          int* flag) {
+  constexpr int nseg = NT / L;
+  const int seg = threadIdx.x / L, lane = threadIdx.x % L;
+  const int B = (nc + 1) / 2;
+  const double tol2 = tol * tol;
+  if (threadIdx.x == 0) *flag = 0;
+  __syncthreads();
+  bool rotated = false;
+  for (int k = seg; k < B; k += nseg) {
+    Cols2<R> b;
+    load_cols<L>(b, X, W, 2 * k, nc, n, ld, lane);
+    double al = norm2<L>(b.x[0]), be = norm2<L>(b.x[1]), ga = 0.0;
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        al += x[r] * x[r];
-        be += y[r] * y[r];
-        ga += x[r] * y[r];
+    for (int r = 0; r < R; ++r) ga += b.x[0][r] * b.x[1][r];
+    ga = add_row<L>(seg_sum(ga));
+    double c, s;
+    bool cancel;
+    if (jacobi_angle(al, be, ga, tol2, c, s, cancel)) {  // the same bits in the whole segment
+      rotate_cols(b.x[0], b.x[1], c, s);
+      rotate_cols(b.w[0], b.w[1], c, s);
+      if (cancel) {
+        al = norm2<L>(b.x[0]);
+        be = norm2<L>(b.x[1]);
       }
-      al = seg_sum(al);
-      be = seg_sum(be);
-      ga = seg_sum(ga);
-      double c, s;
-      if (jacobi_cs(al, be, ga, tol, c, s)) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int i = lane + L * r;
-          const double xn = c * x[r] - s * y[r];
-          if (i < m) aq[i] = s * x[r] + c * y[r];
-          x[r] = xn;
+      store_cols<L>(b, X, W, 2 * k, nc, n, ld, lane);
+      rotated = true;
+    }
+    if (lane == 0) {
+      nn[2 * k] = al;
+      nn[2 * k + 1] = be;
+    }
+  }
+  __syncthreads();
+  for (int d = 0; (1 << d) < B; ++d) {
+    const int hmax = (B + (2 << d) - 1) >> (d + 1);
+    for (int base = 0; base < (hmax << d); base += nseg) {
+      const int k = base + seg, rg = k / hmax, idx = k % hmax;
+      int lo = 0, hi = B;
+      for (int b = d - 1; b >= 0; --b) {
+        const int mid = lo + (hi - lo + 1) / 2;
+        if ((rg >> b) & 1) lo = mid;
+        else hi = mid;
+      }
+      const int mid = lo + (hi - lo + 1) / 2, hp = mid - lo, hq = hi - mid;
+      const bool act = rg < (1 << d) && idx < hp && hq > 0;
+      Cols2<R> P;
+      const int pc = 2 * (lo + idx);
+      if (act) {
+        load_cols<L>(P, X, W, pc, nc, n, ld, lane);
+        P.nn[0] = nn[pc];
+        P.nn[1] = nn[pc + 1];
+      }
+      bool any = false;
+      for (int t = 0; t < hmax; ++t) {
+        if (act && t < hp) {
+          int j = idx + t;
+          if (j >= hp) j -= hp;
+          if (j < hq) {
+            const int qc = 2 * (mid + j);
+            Cols2<R> Q;
+            load_cols<L>(Q, X, W, qc, nc, n, ld, lane);
+            Q.nn[0] = nn[qc];
+            Q.nn[1] = nn[qc + 1];
+            if (rotate_blocks<L>(P, Q, tol2, lane)) {
+              store_cols<L>(Q, X, W, qc, nc, n, ld, lane);
+              if (lane < 2) nn[qc + lane] = lane ? Q.nn[1] : Q.nn[0];
+              any = true;
+            }
+          }
         }
+        __syncthreads();
+      }
+      if (act && any) {
+        store_cols<L>(P, X, W, pc, nc, n, ld, lane);
+        if (lane < 2) nn[pc + lane] = lane ? P.nn[1] : P.nn[0];
+        rotated = true;
+      }
+      __syncthreads();
+    }
+  }
+  if (rotated) *flag = 1;
+  __syncthreads();
+  const bool ret = *flag != 0;
+  __syncthreads();  // every thread has read the flag before it is reused
+  return ret;
+}
+
+// all sweeps of an n x n matrix (n <= SVD_LDS_N) in one workgroup, X and W in LDS
+__global__ __launch_bounds__(SVD_NT_LDS) void k_jacobi_lds(const SvdGroup* __restrict__ groups,
+                                                           const int32_t* __restrict__ which,
+                                                           double* __restrict__ work, int32_t* __restrict__ sweeps) {
+  __shared__ double lds[2 * SVD_LDS_N * (SVD_LDS_N + 8)];
+  __shared__ double nn[SVD_LDS_N + 2];
+  __shared__ int flag;
+  const SvdGroup g = groups[which[blockIdx.x]];
+  const int n = g.n, tid = threadIdx.x;
+  // leading dimension 8 mod 16: the 16-lane segments of a wave read 2-column
+  // blocks that start in different halves of the banks
+  const int ld = ((n + 7) & ~15) + 8;
+  double* X = lds;
+  double* W = lds + n * ld;
+  const int wave = tid >> 6, wl = tid & 63;
+  for (int j = wave; j < n; j += SVD_NT_LDS / 64)
+    for (int i = wl; i < n; i += 64) {
+      X[j * ld + i] = work[g.x + j * n + i];
+      W[j * ld + i] = i == j ? 1.0 : 0.0;
+    }
+  __syncthreads();
+  int sw = 0;
+  for (; sw < SVD_MAX_SWEEPS; ++sw) {
+    const double tol = jacobi_tol(n, sw);
+    bool any;
+    switch ((n + 15) / 16) {
+      case 1: any = sweep_lds<SVD_NT_LDS, SVD_SEG, 1>(X, W, nn, n, n, ld, tol, &flag); break;
+      case 2: any = sweep_lds<SVD_NT_LDS, SVD_SEG, 2>(X, W, nn, n, n, ld, tol, &flag); break;
+      case 3: any = sweep_lds<SVD_NT_LDS, SVD_SEG, 3>(X, W, nn, n, n, ld, tol, &flag); break;
+      case 4: any = sweep_lds<SVD_NT_LDS, SVD_SEG, 4>(X, W, nn, n, n, ld, tol, &flag); break;
+      case 5: any = sweep_lds<SVD_NT_LDS, SVD_SEG, 5>(X, W, nn, n, n, ld, tol, &flag); break;
+      default: any = sweep_lds<SVD_NT_LDS, SVD_SEG, 6>(X, W, nn, n, n, ld, tol, &flag); break;
+    }
+    if (!any) break;
+  }
+  for (int j = wave; j < n; j += SVD_NT_LDS / 64)
+    for (int i = wl; i < n; i += 64) {
+      work[g.x + j * n + i] = X[j * ld + i];
+      work[g.w + j * n + i] = W[j * ld + i];
+    }
+  if (tid == 0) sweeps[blockIdx.x] = sw;
+}
+
+// contiguous columns of X and W between memory and LDS, up to 16 loads in
+// flight per thread
+template <int NT>
+__device__ __forceinline__ void copy_cols(double* __restrict__ dx, double* __restrict__ dw,
+                                          const double* __restrict__ sx, const double* __restrict__ sw, int n) {
+  for (int e0 = threadIdx.x; e0 < n; e0 += 8 * NT) {
+    double v[8], w[8];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int i = lane + L * r;
-          z[r] = i < n ? vq[i] : 0.0;
-        }
+    for (int u = 0; u < 8; ++u) {
+      const bool in = e0 + u * NT < n;
+      v[u] = in ? sx[e0 + u * NT] : 0.0;
+      w[u] = in ? sw[e0 + u * NT] : 0.0;
+    }
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int i = lane + L * r;
-          const double un = c * u[r] - s * z[r];
-          if (i < n) vq[i] = s * u[r] + c * z[r];
-          u[r] = un;
-        }
-        if (lane == 0) *flag = 1;
+    for (int u = 0; u < 8; ++u)
+      if (e0 + u * NT < n) {
+        dx[e0 + u * NT] = v[u];
+        dw[e0 + u * NT] = w[u];
+      }
+  }
+}
+
+// the column blocks P (registers, one 2-column block per segment) against Q (LDS)
+template <int L, int R>
+__device__ __forceinline__ bool cross_blocks(double* __restrict__ Xp, double* __restrict__ Wp, int np,
+                                             const double* __restrict__ gx, const double* __restrict__ gw, double* Xq,
+                                             double* Wq, double* nn, int nq, int n, double tol) {
+  const int seg = threadIdx.x / L, lane = threadIdx.x % L;
+  const int hp = (np + 1) / 2, hq = (nq + 1) / 2, h = hp > hq ? hp : hq;
+  const double tol2 = tol * tol;
+  Cols2<R> P{};
+  if (seg < hp) {  // hp <= NT / L, checked by the host
+    load_cols<L>(P, Xp, Wp, 2 * seg, np, n, n, lane);
+  }
+  copy_cols<SVD_NT_CROSS>(Xq, Wq, gx, gw, nq * n);
+  P.nn[0] = norm2<L>(P.x[0]);
+  P.nn[1] = norm2<L>(P.x[1]);
+  __syncthreads();
+  if (seg < hq) {
+    for (int c = 2 * seg; c < 2 * seg + 2; ++c) {
+      double s = 0.0;
+      for (int i = lane; i < n && c < nq; i += L) s += Xq[c * n + i] * Xq[c * n + i];
+      s = add_row<L>(seg_sum(s));
+      if (lane == 0) nn[c] = s;
+    }
+  }
+  __syncthreads();
+  bool any = false;
+  for (int t = 0; t < h; ++t) {
+    int j = seg + t;
+    if (j >= h) j -= h;
+    if (seg < hp && j < hq) {
+      Cols2<R> Q;
+      load_cols<L>(Q, Xq, Wq, 2 * j, nq, n, n, lane);
+      Q.nn[0] = nn[2 * j];
+      Q.nn[1] = nn[2 * j + 1];
+      if (rotate_blocks<L>(P, Q, tol2, lane)) {
+        store_cols<L>(Q, Xq, Wq, 2 * j, nq, n, n, lane);
+        if (lane < 2) nn[2 * j + lane] = lane ? Q.nn[1] : Q.nn[0];
+        any = true;
       }
     }
     __syncthreads();
   }
-  if (own) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int i = lane + L * r;
-      if (i < m) ap[i] = x[r];
-      if (i < n) vp[i] = u[r];
-    }
-  }
-  __syncthreads();
-  const bool any = *flag != 0;
-  __syncthreads();  // every thread has read the flag before it is reused
+  if (any) store_cols<L>(P, Xp, Wp, 2 * seg, np, n, n, lane);
   return any;
 }
 
-// the variant for column length m (NT threads; 512 leave the registers for
-// 32 elements per lane)
-template <int NT, bool CROSS>
-__device__ __forceinline__ bool jacobi_pairs_m(double* A, double* V, int np, int nq, int m, int n, double tol,
-                                               int* flag) {
-  if constexpr (CROSS && NT <= 512) {
-    if (np <= NT / SVD_SEG) {
-      if (m <= 64) return jacobi_cross_reg<NT, 4>(A, V, np, nq, m, n, tol, flag);
-      if (m <= 128) return jacobi_cross_reg<NT, 8>(A, V, np, nq, m, n, tol, flag);
-      if (m <= 256) return jacobi_cross_reg<NT, 16>(A, V, np, nq, m, n, tol, flag);
-    }
-  }
-  if (m <= 16) return jacobi_pairs<NT, 1, CROSS>(A, V, np, nq, m, n, tol, flag);
-  if (m <= 32) return jacobi_pairs<NT, 2, CROSS>(A, V, np, nq, m, n, tol, flag);
-  if (m <= 64) return jacobi_pairs<NT, 4, CROSS>(A, V, np, nq, m, n, tol, flag);
-  if (m <= 128) return jacobi_pairs<NT, 8, CROSS>(A, V, np, nq, m, n, tol, flag);
-  if (m <= 256) return jacobi_pairs<NT, 16, CROSS>(A, V, np, nq, m, n, tol, flag);
-  if constexpr (NT <= 512)
-    if (m <= 512) return jacobi_pairs<NT, 32, CROSS>(A, V, np, nq, m, n, tol, flag);
-  return jacobi_pairs<NT, 0, CROSS>(A, V, np, nq, m, n, tol, flag);
-}
-
-// zero-padded group matrices: block e (d1 x d2, column-major) goes to
-// row i0, column j0 of its matrix (leading dim ld), transposed when trans
-__global__ __launch_bounds__(256) void k_svd_gather(const SvdGather* __restrict__ items, const double* __restrict__ src,
-                                                    double* __restrict__ work) {
-  const SvdGather it = items[blockIdx.x];
-  const int64_t n = (int64_t)it.d1 * it.d2;
-  for (int64_t e = threadIdx.x; e < n; e += 256) {
-    const int64_t i = e % it.d1, j = e / it.d1;
-    const int64_t d = it.trans ? it.dst_off + j + i * it.ld : it.dst_off + i + j * it.ld;
-    work[d] = src[it.src_off + e] * it.scale;
-  }
-}
-
-__global__ __launch_bounds__(SVD_NT) void k_jacobi_svd(const SvdItem* __restrict__ items, double* __restrict__ work,
-                                                       double* __restrict__ sig, int32_t* __restrict__ sweeps) {
-  __shared__ double lds[SVD_LDS_DOUBLES];
-  __shared__ int rotated;
-  const SvdItem it = items[blockIdx.x];
-  const int m = it.m, n = it.n;  // m >= n >= 1
-  const int tid = threadIdx.x;
-  // LDS only (m*n + n*n <= SVD_LDS_DOUBLES, checked by the host), so that
-  // every access is an LDS instruction
-  double* A = lds;
-  double* V = lds + (int64_t)m * n;
-  for (int64_t e = tid; e < (int64_t)m * n; e += SVD_NT) A[e] = work[it.a_off + e];
-  for (int64_t e = tid; e < (int64_t)n * n; e += SVD_NT) V[e] = (e % (n + 1)) == 0 ? 1.0 : 0.0;
-  __syncthreads();
-
-  const int seg = tid / SVD_SEG, lane = tid % SVD_SEG;
-  constexpr int nseg = SVD_NT / SVD_SEG;
-  int sw = 0;
-  for (; sw < SVD_MAX_SWEEPS; ++sw)
-    if (!jacobi_pairs_m<SVD_NT, false>(A, V, n, 0, m, n, jacobi_tol(m, sw), &rotated)) break;
-  // sigma_j = |a_j|, u_j = a_j / sigma_j (a zero column stays zero)
-  for (int j = seg; j < n; j += nseg) {
-    double* aj = A + (int64_t)j * m;
-    double s2 = 0.0;
-    for (int i = lane; i < m; i += SVD_SEG) s2 += aj[i] * aj[i];
-    s2 = seg_sum(s2);
-    const double sg = sqrt(s2);
-    const double inv = sg > 0.0 ? 1.0 / sg : 0.0;
-    for (int i = lane; i < m; i += SVD_SEG) aj[i] *= inv;
-    if (lane == 0) sig[it.s_off + j] = sg;
-  }
-  __syncthreads();
-  for (int64_t e = tid; e < (int64_t)m * n; e += SVD_NT) work[it.a_off + e] = A[e];
-  for (int64_t e = tid; e < (int64_t)n * n; e += SVD_NT) work[it.v_off + e] = V[e];
-  if (tid == 0) sweeps[blockIdx.x] = sw;
+// one round of a sweep of a matrix with SVD_LDS_N < n <= SVD_QR_MAX_N: the
+// pairs within column block P (q0 == q1) or the pairs of P against Q;
+// rot[sweep * ngroups + grp] is set when one rotated.  A group that rotated
+// nothing in the sweep before is done.  Blocks of 16 columns with 32 lanes a
+// segment (21 us a launch, n = 187) against 32 columns with 16 lanes (51 us, half
+// as many launches): one wave per SIMD either way, so the issue of a step's
+// updates bounds a round, and smaller blocks spread it over more CUs.
+__global__ __launch_bounds__(SVD_NT_CROSS) void k_jacobi_cross(const SvdGroup* __restrict__ groups, int ngroups,
+                                                               const SvdBlockStep* __restrict__ steps,
+                                                               double* __restrict__ work, int32_t* __restrict__ rot,
+                                                               int sweep) {
+  __shared__ double lds[2 * SVD_CROSS_COLS * SVD_QR_MAX_N];
+  __shared__ double nn[SVD_CROSS_COLS + 2];
+  __shared__ int flag;
+  const SvdBlockStep st = steps[blockIdx.x];
+  if (sweep > 0 && rot[(sweep - 1) * ngroups + st.grp] == 0) return;
+  const SvdGroup g = groups[st.grp];
+  const int n = g.n;
+  const bool cross = st.q1 > st.q0;
+  const int c0 = cross ? st.q0 : st.p0, nc = cross ? st.q1 - st.q0 : st.p1 - st.p0;
+  double* X = lds;
+  double* W = lds + nc * n;
+  double* gx = work + g.x + (int64_t)c0 * n;
+  double* gw = work + g.w + (int64_t)c0 * n;
+  double* px = work + g.x + (int64_t)st.p0 * n;
+  double* pw = work + g.w + (int64_t)st.p0 * n;
+  const int np = st.p1 - st.p0;
+  const double tol = jacobi_tol(n, sweep);
+  bool any;
+#define QSX_CROSS(R)                                                                              \
+  any = cross ? cross_blocks<SVD_SEG_CROSS, R>(px, pw, np, gx, gw, X, W, nn, nc, n, tol)          \
+              : (copy_cols<SVD_NT_CROSS>(X, W, gx, gw, nc * n), __syncthreads(), false) ||        \
+                    sweep_lds<SVD_NT_CROSS, SVD_SEG_CROSS, R>(X, W, nn, nc, n, n, tol, &flag)
+  if (n <= 128) QSX_CROSS(4);
+  else if (n <= 160) QSX_CROSS(5);
+  else if (n <= 192) QSX_CROSS(6);
+  else if (n <= 224) QSX_CROSS(7);
+  else QSX_CROSS(8);
+#undef QSX_CROSS
+  any = __syncthreads_or(any);
+  if (!any) return;
+  copy_cols<SVD_NT_CROSS>(gx, gw, X, W, nc * n);
+  if (threadIdx.x == 0) rot[sweep * ngroups + st.grp] = 1;
 }
 
 // one step of the block one-sided Jacobi of a group matrix too large for
@@ -463,15 +731,15 @@ __global__ __launch_bounds__(256) void k_svd_init_v(const SvdItem* __restrict__ 
 
 // result block: dst[r + c * rows] = src[src_off + r + col_c * ld] * scale_c
 // over the kept columns (col_c, scale_c) = cols[col0 + c]
-__global__ __launch_bounds__(256) void k_svd_scatter(const SvdScatter* __restrict__ items,
-                                                     const SvdCol* __restrict__ cols, const double* __restrict__ work,
-                                                     double* __restrict__ out) {
+__global__ __launch_bounds__(64) void k_svd_scatter(const SvdScatter* __restrict__ items,
+                                                    const SvdCol* __restrict__ cols, const double* __restrict__ work,
+                                                    double* __restrict__ out) {
   const SvdScatter it = items[blockIdx.x];
-  const int64_t n = (int64_t)it.rows * it.ncols;
-  for (int64_t e = threadIdx.x; e < n; e += 256) {
-    const int64_t r = e % it.rows, c = e / it.rows;
+  for (int c = blockIdx.y; c < it.ncols; c += gridDim.y) {
     const SvdCol col = cols[it.col0 + c];
-    out[it.dst_off + e] = work[it.src_off + r + (int64_t)col.col * it.ld] * col.scale * it.scale;
+    const double* x = work + it.src_off + (int64_t)col.col * it.ld;
+    for (int r = threadIdx.x; r < it.rows; r += 64)
+      out[it.dst_off + r + (int64_t)c * it.rows] = x[r] * col.scale * it.scale;
   }
 }
 
@@ -479,14 +747,22 @@ __global__ __launch_bounds__(256) void k_svd_scatter(const SvdScatter* __restric
 
 void launch_svd_gather(const SvdGather* ditems, int nitems, const double* src, double* work, hipStream_t s) {
   if (nitems <= 0) return;
-  hipLaunchKernelGGL(k_svd_gather, dim3(nitems), dim3(256), 0, s, ditems, src, work);
+  hipLaunchKernelGGL(k_svd_gather, dim3(nitems, kColSplit), dim3(64), 0, s, ditems, src, work);
   QSX_HIP(hipGetLastError());
 }
 
-void launch_jacobi_svd(const SvdItem* ditems, int nitems, double* work, double* sig, int32_t* sweeps,
+void launch_jacobi_lds(const SvdGroup* dgroups, const int32_t* dwhich, int n, double* work, int32_t* sweeps,
                        hipStream_t s) {
-  if (nitems <= 0) return;
-  hipLaunchKernelGGL(k_jacobi_svd, dim3(nitems), dim3(SVD_NT), 0, s, ditems, work, sig, sweeps);
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_jacobi_lds, dim3(n), dim3(SVD_NT_LDS), 0, s, dgroups, dwhich, work, sweeps);
+  QSX_HIP(hipGetLastError());
+}
+
+void launch_jacobi_cross(const SvdGroup* dgroups, int ngroups, const SvdBlockStep* dsteps, int nsteps, double* work,
+                         int32_t* rot, int sweep, hipStream_t s) {
+  if (nsteps <= 0) return;
+  hipLaunchKernelGGL(k_jacobi_cross, dim3(nsteps), dim3(SVD_NT_CROSS), 0, s, dgroups, ngroups, dsteps, work, rot,
+                     sweep);
   QSX_HIP(hipGetLastError());
 }
 
@@ -515,7 +791,7 @@ void launch_svd_init_v(const SvdItem* dgroups, const int32_t* dwhich, int n, dou
 void launch_svd_scatter(const SvdScatter* ditems, int nitems, const SvdCol* dcols, const double* work, double* out,
                         hipStream_t s) {
   if (nitems <= 0) return;
-  hipLaunchKernelGGL(k_svd_scatter, dim3(nitems), dim3(256), 0, s, ditems, dcols, work, out);
+  hipLaunchKernelGGL(k_svd_scatter, dim3(nitems, kColSplit), dim3(64), 0, s, ditems, dcols, work, out);
   QSX_HIP(hipGetLastError());
 }
 

@@ -159,3 +159,54 @@ def test_ortho_rank_deficient_groups(gpu):
         num = sum(float(np.sum((a - b) ** 2)) for a, b in zip(X.data, XR.data))
         den = sum(float(np.sum(b * b)) for b in XR.data)
         assert np.sqrt(num / den) < 1e-12
+
+
+# group matrices (rows, columns) at the edges of the SVD's paths: panels of 16
+# columns, the in-LDS / column-block line (n = 96 / 97), register rows of the
+# cross rounds (multiples of 32), row buckets of the QR (256, 512, 1024 rows)
+# and the line beyond which the matrix itself is swept (n = 257, m = 1025)
+SHAPES = [(1, 1), (2, 2), (5, 2), (16, 16), (17, 16), (40, 17), (33, 32), (96, 96), (97, 97), (130, 96), (128, 97),
+          (129, 128), (140, 129), (256, 193), (257, 225), (256, 256), (513, 60), (600, 100), (1024, 33), (1025, 20),
+          (258, 257), (300, 1)]
+
+
+@pytest.mark.parametrize("kind", ["random", "graded", "deficient", "scaled"])
+@pytest.mark.parametrize("wide", [False, True])
+def test_svd_shapes(gpu, kind, wide):
+    """singular values, A1 . A2 = psi and the isometry of A1 over the shapes
+    where the decomposition changes path; graded: values over six decades,
+    deficient: half the columns repeated and one zero, scaled: entries near
+    2^+-400.  Tolerance: an element takes about n rotations a sweep, over at
+    most 10 sweeps of a preconditioned matrix and 60 (the limit) of one swept
+    as it is, each rounding at 2 eps of its row: a random walk of
+    2 sqrt(sweeps (m + n)) eps, times 4."""
+    rng = np.random.default_rng(23 + wide)
+    for k, (m, n) in enumerate(SHAPES):
+        if kind == "deficient" and n > 256:
+            continue  # without the QRs the sweeps of half-rank columns do not end
+        if kind == "graded":
+            M = (rng.standard_normal((m, n)) / np.sqrt(m) * np.exp(-14.0 * np.arange(n) / n)) @ \
+                (rng.standard_normal((n, n)) / np.sqrt(n))
+        else:
+            M = rng.standard_normal((m, n))
+        if kind == "deficient":
+            M[:, n // 2:] = M[:, :n - n // 2]
+            M[:, -1] = 0.0
+        if kind == "scaled":
+            M = np.ldexp(M, 400 if k % 2 else -400)
+        if wide:
+            M = M.T
+        P = Q.QSpace([np.array([[0]]), np.array([[0]])], [M], "A", ["L", "R*"])
+        print(kind, M.shape, flush=True)
+        A1, A2, info = Q.orthoQS(P, 1, stol=0.0)
+        s = np.linalg.svd(M, compute_uv=False)
+        tol = 8.0 * np.sqrt((60.0 if n > 256 or m > 1024 else 10.0) * (m + n)) * np.finfo(float).eps
+        assert np.abs(info["svd"] - s).max() <= tol * max(s[0], 1e-300)
+        if not A2.nblk:
+            assert s[0] == 0.0
+            continue
+        U, V = A1.data[0], A2.data[0]
+        # A2 is (R, new): psi = U V^T
+        assert np.linalg.norm(U @ V.T - M) <= tol * np.linalg.norm(M)
+        if kind != "deficient":  # columns of zero singular values are zero
+            assert np.abs(U.T @ U - np.eye(n)).max() <= tol
