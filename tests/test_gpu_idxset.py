@@ -87,3 +87,28 @@ def test_hpsi_heis4000_matches_oracle(gpu, heis4000):
     H.autotune(reps=3)
     got = H.apply(x)
     assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < TOL
+
+
+def _labelled(na, nb, nlab, seed, ka=1, kb=1):
+    """two rank-(1 + k) U(1) tensors of 1x..x1 blocks with na and nb distinct
+    records over nlab contracted labels, in random order"""
+    rng = np.random.RandomState(seed)
+
+    def make(n, k, tag):
+        c = rng.permutation(np.arange(n) % nlab)
+        rec = np.stack([c] + [rng.permutation(n) if j == 0 else rng.randint(-3, 4, n) for j in range(k)], axis=1)
+        return Q.QSpace([rec[:, j:j + 1] for j in range(1 + k)], [np.ones((1,) * (1 + k))] * n, "A",
+                        ["x" if tag == "A" else "x*"] + [f"{tag}{j}" for j in range(k)])
+
+    return make(na, ka, "A"), make(nb, kb, "B")
+
+
+# (records of A, of B, distinct contracted labels): one pair; the sizes of the
+# one-launch engine and one beyond (1024 records, 2048 pairs); many-to-many
+@pytest.mark.parametrize("na,nb,nlab", [(1, 1, 1), (3, 2, 4), (63, 65, 9), (64, 64, 2), (1024, 1024, 512), (1025, 40, 600),
+                                        (40, 1025, 600), (64, 32, 1), (2049, 1, 1), (683, 3, 1), (1024, 1024, 1024)])
+def test_idxset_engine_sizes(gpu, na, nb, nlab):
+    A, B = _labelled(na, nb, nlab, seed=na + 7 * nb)
+    _compare(A, [0], B, [0])
+    A, B = _labelled(na, nb, nlab, seed=na + 7 * nb + 1, ka=2, kb=3)
+    _compare(A, [0], B, [0])
