@@ -45,24 +45,31 @@ static WorkList build_wave_work(const std::vector<WorkTarget>& targets, const st
   int G = maxf <= 2 ? pol.group_waves : 4;
   while (G > 4 && G * maxf * maxf > 16) G /= 2;
   out.wg_waves = G;
-  struct WG {
+  // a workgroup whose G waves share a tile (items gi[first .. first+G-1]) or a
+  // one-wave item (si[first]); the orders below move these and not the items
+  struct Ref {
     double cost;
     int64_t key;  // locality key: the larger operand's block of the target's first pair
-    std::vector<WorkItem> it;
+    size_t first;
   };
-  struct Solo {
-    double cost;
-    int64_t key;
-    WorkItem w;
-  };
-  std::vector<WG> groups;   // workgroups of 4 tasks of one tile
-  std::vector<Solo> solo;   // one-wave items
+  std::vector<WorkItem> gi, si;
+  std::vector<Ref> groups, solo;
+  std::vector<int64_t> cum;  // k-steps before each pair of the target
+  size_t ntiles = 0;
+  for (const WorkTarget& t : targets)
+    if (t.M > 0 && t.N > 0) {
+      const size_t mf = (t.M + 15) / 16, nf = (t.N + 15) / 16;
+      ntiles += ((mf + maxf - 1) / maxf) * ((nf + maxf - 1) / maxf);
+    }
+  si.reserve(ntiles);
+  solo.reserve(ntiles);
   int64_t slot = 0;
   for (const WorkTarget& t : targets) {
     const int M = t.M, N = t.N;
     if (M <= 0 || N <= 0) continue;
     int64_t steps = 0;
-    for (int64_t p = t.p0; p < t.p1; ++p) steps += (pairs[p].K + WKS - 1) / WKS;
+    cum.assign(1, 0);
+    for (int64_t p = t.p0; p < t.p1; ++p) cum.push_back(steps += (pairs[p].K + WKS - 1) / WKS);
     const int mf = (M + 15) / 16, nf = (N + 15) / 16;
     const int ntm = (mf + maxf - 1) / maxf, ntn = (nf + maxf - 1) / maxf;
     int64_t key = -1;
@@ -78,18 +85,10 @@ static WorkList build_wave_work(const std::vector<WorkTarget>& targets, const st
         w.p1 = -1;
         return w;
       }
-      auto locate = [&](int64_t s, int& p, int& k) {
-        for (int64_t q = t.p0; q < t.p1; ++q) {
-          const int64_t n = (pairs[q].K + WKS - 1) / WKS;
-          if (s < n) {
-            p = (int)q;
-            k = (int)(s * WKS);
-            return;
-          }
-          s -= n;
-        }
-        p = (int)t.p1;
-        k = 0;
+      auto locate = [&](int64_t s, int& p, int& k) {  // s < steps
+        const int64_t q = std::upper_bound(cum.begin(), cum.end(), s) - cum.begin() - 1;
+        p = (int)(t.p0 + q);
+        k = (int)((s - cum[q]) * WKS);
       };
       int kb;
       locate(s0, w.p0, w.k0);
@@ -122,17 +121,15 @@ static WorkList build_wave_work(const std::vector<WorkTarget>& targets, const st
           WorkItem w = base;
           if (nch > 1) w.slot = (int32_t)(slot + q);
           if (grp) {
-            WG g;
-            g.key = key;
-            g.cost = per_step * (double)((c1 - c0 + G - 1) / G) + 16.0;
+            groups.push_back({per_step * (double)((c1 - c0 + G - 1) / G) + 16.0, key, gi.size()});
             for (int v = 0; v < G; ++v) {
               WorkItem x = range(w, c0 + (c1 - c0) * v / G, c0 + (c1 - c0) * (v + 1) / G);
               x.group = 1;
-              g.it.push_back(x);
+              gi.push_back(x);
             }
-            groups.push_back(std::move(g));
           } else {
-            solo.push_back({per_step * (double)(c1 - c0) + 8.0, key, range(w, c0, c1)});
+            solo.push_back({per_step * (double)(c1 - c0) + 8.0, key, si.size()});
+            si.push_back(range(w, c0, c1));
           }
         }
         if (nch > 1) {
@@ -159,43 +156,41 @@ static WorkList build_wave_work(const std::vector<WorkTarget>& targets, const st
     int64_t chunks = 0;
     const int fm = (w.shape - SH_WAVE) / 4 + 1, fn = (w.shape - SH_WAVE) % 4 + 1;
     const int ck = 4 * wave_chunk_steps(fm, fn);
-    for (int p = w.p0; p <= w.p1; ++p) {
+    for (int p = w.p0; p <= w.p1 && chunks <= 2; ++p) {
       const int kb = p == w.p0 ? w.k0 : 0, ke = p == w.p1 ? w.k1 : pairs[p].K;
       chunks += (ke - kb + ck - 1) / ck;
     }
     if (chunks <= 2) w.pad |= kShortItem;
   };
-  for (Solo& x : solo) mark_short(x.w);
-  for (WG& g : groups)
-    for (WorkItem& w : g.it) mark_short(w);
-  auto pad_item = []() {
-    WorkItem pad{};
-    pad.slot = -2;
-    pad.p0 = 0;
-    pad.p1 = -1;
-    pad.shape = wave_shape(1, 1);
-    return pad;
-  };
-  auto by_cost = [](const WG& x, const WG& y) { return x.cost > y.cost; };
-  // one bin's workgroups: its group workgroups plus its solo items packed G
-  // to a workgroup longest first (only the bin's last workgroup is padded;
-  // locality lives in the L2 of the bin's XCD, so a workgroup may mix keys)
-  auto pack = [&](std::vector<WG>& wgs, std::vector<Solo>& so) {
-    std::stable_sort(so.begin(), so.end(), [](const Solo& x, const Solo& y) { return x.cost > y.cost; });
-    for (size_t i = 0; i < so.size(); i += G) {
-      WG g;
-      g.cost = so[i].cost;
-      g.key = so[i].key;
-      for (size_t j = i; j < i + G; ++j) g.it.push_back(j < so.size() ? so[j].w : pad_item());
-      wgs.push_back(std::move(g));
-    }
+  for (WorkItem& w : si) mark_short(w);
+  for (WorkItem& w : gi) mark_short(w);
+  WorkItem pad{};
+  pad.slot = -2;
+  pad.p0 = 0;
+  pad.p1 = -1;
+  pad.shape = wave_shape(1, 1);
+  auto by_cost = [](const Ref& x, const Ref& y) { return x.cost > y.cost; };
+  // one bin's workgroups, longest first: its group workgroups plus its solo
+  // items packed G to a workgroup longest first (only the bin's last workgroup
+  // is padded; locality lives in the L2 of the bin's XCD, so a workgroup may
+  // mix keys).  A packed workgroup's first is gi.size() + its place in so.
+  auto pack = [&](std::vector<Ref>& wgs, std::vector<Ref>& so) {
+    std::stable_sort(so.begin(), so.end(), by_cost);
+    for (size_t i = 0; i < so.size(); i += G) wgs.push_back({so[i].cost, so[i].key, gi.size() + i});
     std::stable_sort(wgs.begin(), wgs.end(), by_cost);
+  };
+  auto emit = [&](const Ref& wg, const std::vector<Ref>& so) {
+    if (wg.first < gi.size()) {
+      out.items.insert(out.items.end(), gi.begin() + wg.first, gi.begin() + wg.first + G);
+      return;
+    }
+    for (size_t j = wg.first - gi.size(), e = j + G; j < e; ++j)
+      out.items.push_back(j < so.size() ? si[so[j].first] : pad);
   };
   const int nbins = pol.xcd_bins;
   if (nbins <= 1) {
     pack(groups, solo);
-    for (const WG& g : groups)
-      for (const WorkItem& w : g.it) out.items.push_back(w);
+    for (const Ref& g : groups) emit(g, solo);
   } else {
     // XCD-aware order: workgroup i runs on XCD i % nbins (round-robin
     // dispatch), each XCD with its own L2.  The work of one locality key
@@ -206,18 +201,17 @@ static WorkList build_wave_work(const std::vector<WorkTarget>& targets, const st
     // empty workgroups).
     struct Key {
       double cost = 0;
-      std::vector<WG> wgs;
-      std::vector<Solo> so;
+      std::vector<Ref> wgs, so;
     };
     std::map<int64_t, Key> bykey;
     double total = 0;
-    for (WG& g : groups) {
+    for (const Ref& g : groups) {
       total += g.cost;
       Key& k = bykey[g.key];
       k.cost += g.cost;
-      k.wgs.push_back(std::move(g));
+      k.wgs.push_back(g);
     }
-    for (Solo& x : solo) {
+    for (const Ref& x : solo) {
       const double c = x.cost / G;  // a solo item is one wave of a workgroup
       total += c;
       Key& k = bykey[x.key];
@@ -227,21 +221,20 @@ static WorkList build_wave_work(const std::vector<WorkTarget>& targets, const st
     std::vector<Key*> keys;
     for (auto& kv : bykey) keys.push_back(&kv.second);
     std::stable_sort(keys.begin(), keys.end(), [](const Key* x, const Key* y) { return x->cost > y->cost; });
-    std::vector<std::vector<WG>> bins(nbins);
-    std::vector<std::vector<Solo>> bsolo(nbins);
+    std::vector<std::vector<Ref>> bins(nbins), bsolo(nbins);
     std::vector<double> load(nbins, 0.0);
     const double share = total / nbins;
     auto least = [&]() { return (int)(std::min_element(load.begin(), load.end()) - load.begin()); };
     for (Key* k : keys) {
       if (k->cost > share) {
         std::stable_sort(k->wgs.begin(), k->wgs.end(), by_cost);
-        for (WG& g : k->wgs) {
+        for (const Ref& g : k->wgs) {
           const int b = least();
           load[b] += g.cost;
-          bins[b].push_back(std::move(g));
+          bins[b].push_back(g);
         }
-        std::stable_sort(k->so.begin(), k->so.end(), [](const Solo& x, const Solo& y) { return x.cost > y.cost; });
-        for (Solo& x : k->so) {
+        std::stable_sort(k->so.begin(), k->so.end(), by_cost);
+        for (const Ref& x : k->so) {
           const int b = least();
           load[b] += x.cost / G;
           bsolo[b].push_back(x);
@@ -249,8 +242,8 @@ static WorkList build_wave_work(const std::vector<WorkTarget>& targets, const st
       } else {
         const int b = least();
         load[b] += k->cost;
-        for (WG& g : k->wgs) bins[b].push_back(std::move(g));
-        for (Solo& x : k->so) bsolo[b].push_back(x);
+        bins[b].insert(bins[b].end(), k->wgs.begin(), k->wgs.end());
+        bsolo[b].insert(bsolo[b].end(), k->so.begin(), k->so.end());
       }
     }
     size_t depth = 0;
@@ -258,13 +251,11 @@ static WorkList build_wave_work(const std::vector<WorkTarget>& targets, const st
       pack(bins[b], bsolo[b]);
       depth = std::max(depth, bins[b].size());
     }
+    out.items.reserve(depth * nbins * G);
     for (size_t r = 0; r < depth; ++r)
       for (int b = 0; b < nbins; ++b) {
-        if (r < bins[b].size()) {
-          for (const WorkItem& w : bins[b][r].it) out.items.push_back(w);
-        } else {
-          for (int v = 0; v < G; ++v) out.items.push_back(pad_item());
-        }
+        if (r < bins[b].size()) emit(bins[b][r], bsolo[b]);
+        else out.items.insert(out.items.end(), G, pad);
       }
   }
   for (WorkItem& w : out.items) {
