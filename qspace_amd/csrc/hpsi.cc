@@ -258,6 +258,56 @@ static void hpsi_build_work(HpsiPlan& H) {
   }
 }
 
+// The decomposition of an untuned plan, from each stage's size: M, its MFMAs
+// (16x16 fragments x k-steps of 4; M / 1024 a SIMD on average), and the longest
+// tile's k-steps.  Too little work for the chip: tiles are shared by the waves
+// of a workgroup down to few MFMAs a wave; enough: fewer, larger items.  us per
+// H*psi of the stage's alternatives, other stage as before, operators taken in
+// turn (cold):
+//  stage 1, sharing tiles beyond 16 / 32 / 64 MFMAs: M = 2.9e3 (Heisenberg D* =
+//    300) 19.3 / 20.3 / 21.6; 1.3e4 (1000) 23.3 / 22.9 / 25.0; 3.0e4 (2000) 27.4
+//    / 27.2 / 28.2; 4.3e4 (pseudo-MPO 1500) 35.5 / 34.3 / 34.5; 5.4e4 (3000) 34.2
+//    / 32.4 / 31.6; 2.7e5 (16000) 95.0 / 90.5 / 88.3
+//  stage 2, T . R into psi's ragged blocks, in 16x16 tiles shared beyond 16 / 64
+//    MFMAs: M = 900 (300) 17.7 / 21.7; k-ranges split beyond 48 / 256 MFMAs where
+//    the longest tile, over four waves, is longer than 1.5 average SIMDs: 1.5e4
+//    (1000) 23.6 / 25.1, 3.6e4 (2000) 27.1 / 28.4, 7.6e4 (Hubbard 1500) 36.3 /
+//    39.1, 7.8e4 (pseudo 1500) 33.0 / 34.7, but where it is not 7.8e4 (4000) 37.8 /
+//    36.9
+//  stage 2, 2x2-fragment tiles (split beyond 96 MFMAs by the same measure) /
+//    16x16 tiles: 1.1e5 (pseudo 4000) 39.1 / 40.1, 1.1e5 (Hubbard 2500) 38.2 /
+//    39.8, 1.9e5 (Hubbard 4000) 53.7 / 57.6, 1.9e5 (12000) 62.9 / 70.7, 2.5e5
+//    (16000) 75.8 / 88.5; but 1.3e5 with short k-ranges (8000) 46.3 / 45.7
+static void default_policy(const std::vector<WorkTarget>& targets, const std::vector<PairDesc>& pairs, int stage,
+                           WorkPolicy& pol) {
+  double mfma = 0, longest = 0;
+  for (const WorkTarget& t : targets) {
+    double steps = 0;
+    for (int64_t p = t.p0; p < t.p1; ++p) steps += (pairs[p].K + 3) / 4;
+    mfma += steps * ((t.M + 15) / 16) * ((t.N + 15) / 16);
+    longest = std::max(longest, steps);
+  }
+  const double mean = mfma / 1024;  // MFMAs per SIMD
+  pol.split_mfma = 256;
+  if (stage == 0) {
+    pol.wave_max = 2;
+    pol.group_mfma = mean < 8 ? 16 : mean < 44 ? 32 : 64;
+    return;
+  }
+  if (mean >= 150 || (mean >= 100 && longest / 4 > mean)) {
+    pol.wave_max = 2;
+    pol.group_mfma = 16;
+    if (longest > 1.5 * mean) pol.split_mfma = 96;  // 4 fragments over 4 waves
+  } else {
+    pol.wave_max = 1;
+    pol.group_mfma = mean < 8 ? 16 : 64;
+    if (mean >= 8 && longest / 4 > 1.5 * mean) {
+      pol.group_mfma = 16;
+      pol.split_mfma = 48;
+    }
+  }
+}
+
 // ---------------------------------------------------------------- autotuner
 // Tile shapes and k-splits come from timing candidate work decompositions of
 // each stage on the plan itself (HIP events, median of reps).  The result is
@@ -738,15 +788,6 @@ static void hpsi_create(HpsiPlan& H, const std::vector<const qsx_tensor*>& Ls, c
   if (fermA && Ls.size() != 1) fail(QSX_ERR_ARG, "H*psi: fermion signs need a single left environment");
   H.N = H.psi.total();
   H.pol1.slots = H.pol2.slots = resident_slots();
-  // default decomposition of an untuned plan: the k-range of a wave item
-  // split beyond 256 MFMAs in both stages; stage 2 (T . R into psi's ragged
-  // blocks) in single 16x16 wave tiles.  Measured on the Heisenberg (D* =
-  // 2000, 4000, 8000) and Hubbard (D* = 4000) operators, this is within the
-  // autotuner's timing noise of its choice, where the generic contraction
-  // default (2x2-fragment tiles, no split) left stage 2 up to 1.5x slower.
-  H.pol1.split_mfma = 256;
-  H.pol2.split_mfma = 256;
-  H.pol2.wave_max = 1;
   qsx_opts so{};
   so.mode = QSX_MODE_BATCHED;
   so.verbose = 0;
@@ -1000,6 +1041,8 @@ static void hpsi_create(HpsiPlan& H, const std::vector<const qsx_tensor*>& Ls, c
     H.dpairs2s = alloc_for(H.pairs2s, parts);
     upload_many(parts, s);
   }
+  default_policy(H.targets1, H.pairs1, 0, H.pol1);
+  default_policy(H.targets2, H.pairs2, 1, H.pol2);
   hpsi_build_work(H);
   clk.lap("work lists");
   if (H.mode == QSX_MODE_SPLIT_BF16 || H.mode == QSX_MODE_SPLIT_F32) hpsi_split_setup(H);
