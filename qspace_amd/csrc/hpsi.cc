@@ -1211,20 +1211,34 @@ static void lanczos(HpsiPlan& H, const double* psi0, int niter, double* e0, doub
   vec_normalize_partial(w, V, pa, nullptr, N, s);
   clk.lap("upload psi0");
   // the iteration sequence is launched directly: the host enqueues all
-  // steps while the device runs the earlier ones (5 launches per step)
-  for (int j = 0; j < niter; ++j) {
-    double* vj = V + (int64_t)j * N;
-    eig_hpsi(H, vj, w, s);
-    // full re-orthogonalisation, classical Gram-Schmidt twice; the first
-    // pass's coefficient of v_j is alpha_j = <v_j, H v_j>; the second pass
-    // is fused with the normalisation (beta_j from |w'|^2 - |c'|^2)
-    vec_mdot_partial(V, N, j + 1, w, N, pa, s);
-    vec_gs_update_mdot(w, V, N, pa, j + 1, N, alpha + j, j, V, j + 1, 1, pb, s);
-    vec_gs_update_normalize(w, V, N, pb, j + 1, N, V + (int64_t)(j + 1) * N, beta + j, s);
+  // steps while the device runs the earlier ones (5 launches per step).
+  // Full re-orthogonalisation: for a symmetric H, w = H v_j has components
+  // along v_{j-1} and v_j and rounding along the others, so those two are
+  // subtracted first (their dots read two vectors) and one full Gram-Schmidt
+  // pass, fused with the normalisation (beta_j from |w'|^2 - |c'|^2), does
+  // what the second of two does.  Where a full pass still finds components
+  // above rounding (H not symmetric, or a breakdown), it says so (beta_j < 0)
+  // and the sequence is run again with two full passes a step.  The
+  // coefficient of v_j is alpha_j = <v_j, H v_j>.
+  for (const bool full : {false, true}) {
+    for (int j = 0; j < niter; ++j) {
+      double* vj = V + (int64_t)j * N;
+      eig_hpsi(H, vj, w, s);
+      if (full) {
+        vec_mdot_partial(V, N, j + 1, w, N, 0, pa, s);
+        vec_gs_update_mdot(w, V, N, pa, j + 1, N, alpha + j, j, V, j + 1, 1, pb, s);
+      } else {
+        const int u = std::min(2, j + 1);
+        vec_mdot_partial(V + (int64_t)(j + 1 - u) * N, N, u, w, N, 0, pa, s);
+        vec_gs_local_mdot(w, V, N, pa, u, j + 1, N, alpha + j, pb, s);
+      }
+      vec_gs_update_normalize(w, V, N, pb, j + 1, N, V + (int64_t)(j + 1) * N, beta + j, !full, s);
+    }
+    clk.lap("enqueue the steps");
+    QSX_HIP(hipStreamSynchronize(s));
+    clk.lap("device drain");
+    if (std::none_of(H.hsmall + niter, H.hsmall + 2 * niter, [](double x) { return x < 0.0; })) break;
   }
-  clk.lap("enqueue the steps");
-  QSX_HIP(hipStreamSynchronize(s));
-  clk.lap("device drain");
   std::vector<double> al(H.hsmall, H.hsmall + niter), b(H.hsmall + niter, H.hsmall + 2 * niter);
   b.push_back(0.0);
   // breakdown: a beta_j at rounding level means the Krylov space of psi0
@@ -1303,24 +1317,33 @@ static void davidson(HpsiPlan& H, const double* psi0, int niter, double* e0, dou
     sym_lowest(k, Hk, th, y);
     if (ritz) ritz[it] = th;
     if (e0) *e0 = th;
-    // u = V y and the residual r = H u - theta u in one pass (y and theta
-    // in one host-to-device copy)
     std::copy(y.begin(), y.begin() + k, hy);
     hy[k] = th;
-    QSX_HIP(hipMemcpyAsync(dy, hy, sizeof(double) * (k + 1), hipMemcpyHostToDevice, s));
     if (it + 1 == niter) break;
-    vec_combine_res(u, hu, V, HV, N, dy, k, N, s);
-    // r orthogonalised twice against V and normalised: classical
-    // Gram-Schmidt, the reductions' final sums folded into their consumers,
-    // the second pass fused with the normalisation (|r| to ret[mmax])
-    vec_mdot_partial(V, N, k, hu, N, pa, s);
-    vec_gs_update_mdot(hu, V, N, pa, k, N, nullptr, 0, V, k, 1, pb, s);
-    vec_gs_update_normalize(hu, V, N, pb, k, N, V + (int64_t)k * N, dback + mmax, s);
-    eig_hpsi(H, V + (int64_t)k * N, HV + (int64_t)k * N, s);
+    // the residual r = H V y - theta V y
+    vec_combine_res(hu, V, HV, N, hy, dy, k, N, s);
+    double* vk = V + (int64_t)k * N;
     // grow the projected matrix by one row/column; one host round trip
     // brings the new column and the residual norm
-    vec_mdot(V, N, k + 1, HV + (int64_t)k * N, N, pa, dback, 0, s);
-    QSX_HIP(hipStreamSynchronize(s));
+    auto grow = [&]() {
+      eig_hpsi(H, vk, HV + (int64_t)k * N, s);
+      vec_mdot(V, N, k + 1, HV + (int64_t)k * N, N, pa, dback, 0, s);
+      QSX_HIP(hipStreamSynchronize(s));
+    };
+    // r orthogonalised against V and normalised (|r| to hback[mmax]).  The
+    // Ritz residual is orthogonal to V but for rounding, so one Gram-Schmidt
+    // pass does what the second of two does; where it finds more (|r| near
+    // rounding, H not symmetric) it says so and the step takes two passes,
+    // the reductions' final sums folded into their consumers
+    vec_mdot_partial(V, N, k, hu, N, 1, pa, s);
+    vec_gs_update_normalize(hu, V, N, pa, k, N, vk, dback + mmax, true, s);
+    grow();
+    if (hback[mmax] < 0.0) {
+      vec_mdot_partial(V, N, k, hu, N, 0, pa, s);
+      vec_gs_update_mdot(hu, V, N, pa, k, N, nullptr, 0, V, k, 1, pb, s);
+      vec_gs_update_normalize(hu, V, N, pb, k, N, vk, dback + mmax, false, s);
+      grow();
+    }
     const double* back = hback;
     // converged when the orthogonalised residual is at rounding level
     // relative to the projected matrix (its entries are bounded by |H|):
@@ -1344,7 +1367,8 @@ static void davidson(HpsiPlan& H, const double* psi0, int niter, double* e0, dou
     ++k;
   }
   if (gs) {
-    // the Ritz vector V y (dy holds the last y) back in the caller's basis
+    // the Ritz vector V y (hy holds the last y) back in the caller's basis
+    QSX_HIP(hipMemcpyAsync(dy, hy, sizeof(double) * k, hipMemcpyHostToDevice, s));
     vec_combine(u, V, N, dy, k, N, s, H.dsw);
     eig_download(H, gs, u, s);
   }

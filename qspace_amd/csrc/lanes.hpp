@@ -1,4 +1,4 @@
-// svd_dev.hpp -- device helpers of the block SVD kernels (svd.hip, svdqr.hip)
+// lanes.hpp -- sums and exchanges across a wave's lanes, and 1/sqrt (device)
 #pragma once
 
 #include <hip/hip_runtime.h>

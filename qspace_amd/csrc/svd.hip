@@ -16,7 +16,7 @@
 #include <cfloat>
 
 #include "qsx_internal.hpp"
-#include "svd_dev.hpp"
+#include "lanes.hpp"
 
 namespace qsx {
 namespace {

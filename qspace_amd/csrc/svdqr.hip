@@ -11,7 +11,7 @@
 #include <cfloat>
 
 #include "qsx_internal.hpp"
-#include "svd_dev.hpp"
+#include "lanes.hpp"
 
 namespace qsx {
 namespace {

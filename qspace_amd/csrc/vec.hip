@@ -8,6 +8,7 @@
 
 #include <algorithm>
 
+#include "lanes.hpp"
 #include "qsx_internal.hpp"
 #include "vec.hpp"
 
@@ -18,7 +19,7 @@ constexpr int RT = 256;
 
 __device__ __forceinline__ double block_sum(double v) {
   __shared__ double red[RT / 64];
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  v = wave_sum(v);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (lane == 0) red[w] = v;
   __syncthreads();
@@ -30,21 +31,17 @@ __device__ __forceinline__ double block_sum(double v) {
 }
 
 // the DOT_BLOCKS partials of one reduction summed by one wave (four per
-// lane in a fixed pairing, then a fixed shuffle tree): every block that
+// lane in a fixed pairing, then a fixed tree over the lanes): every block that
 // needs the value sums it in the same order, so all of them hold the same
-// bits
+// bits.  The trees over lanes are DPP and permlane steps, not ds_bpermute
+// (__shfl): the kernels below end in up to 33 of them per wave.
 static_assert(DOT_BLOCKS == 256, "the partial sums read four partials per lane");
 __device__ __forceinline__ double lane_partials(const double* __restrict__ p, int lane) {
   return (p[lane] + p[lane + 64]) + (p[lane + 128] + p[lane + 192]);
 }
-__device__ __forceinline__ double wave_reduce(double s) {
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-  return s;  // valid in lane 0
-}
 // the result is in every lane
 __device__ __forceinline__ double wave_sum_partials(const double* __restrict__ p) {
-  const double s = wave_reduce(lane_partials(p, threadIdx.x & 63));
-  return __shfl(s, 0, 64);
+  return wave_sum(lane_partials(p, threadIdx.x & 63));
 }
 
 // c[j] = sum_b partial[j][b] for j < m, one wave per j; a wave takes up to
@@ -63,7 +60,7 @@ __device__ __forceinline__ void sum_coefficients(const double* __restrict__ part
     }
 #pragma unroll
     for (int q = 0; q < kSumGroup; ++q) {
-      const double s = wave_reduce(v[q]);
+      const double s = wave_sum(v[q]);
       const int j = j0 + q * NW;
       if (lane == 0 && j < m) c[j] = s;
     }
@@ -71,12 +68,13 @@ __device__ __forceinline__ void sum_coefficients(const double* __restrict__ part
   __syncthreads();
 }
 
-// partial[j*DOT_BLOCKS + b] = sum over the b-th slice of V_j . w
-__global__ __launch_bounds__(RT) void k_mdot_partial(const double* __restrict__ V, int64_t ldv,
+// partial[j*DOT_BLOCKS + b] = sum over the b-th slice of V_j . w for j < m, of
+// w . w for j = m
+__global__ __launch_bounds__(RT) void k_mdot_partial(const double* __restrict__ V, int64_t ldv, int m,
                                                       const double* __restrict__ w, int64_t n,
                                                       double* __restrict__ partial) {
   const int j = blockIdx.y, b = blockIdx.x;
-  const double* v = V + (int64_t)j * ldv;
+  const double* v = j < m ? V + (int64_t)j * ldv : w;
   double s = 0;
   for (int64_t i = (int64_t)b * RT + threadIdx.x; i < n; i += (int64_t)DOT_BLOCKS * RT) s += v[i] * w[i];
   s = block_sum(s);
@@ -120,21 +118,36 @@ __global__ __launch_bounds__(RT) void k_combine(double* __restrict__ y, const do
   }
 }
 
-// u = V c, r = HV c - theta u with theta = c[m] (the Davidson Ritz vector
-// and its residual in one pass over V and HV)
-__global__ __launch_bounds__(RT) void k_combine_res(double* __restrict__ u, double* __restrict__ r,
-                                                     const double* __restrict__ V, const double* __restrict__ HV,
-                                                     int64_t ldv, const double* __restrict__ c, int m, int64_t n) {
+// r = HV c - theta V c with theta = c[m] (the residual of the Davidson Ritz
+// vector V c, in one pass over V and HV).  Up to kArgCoef coefficients come as
+// a kernel argument: a copy to the device in front of every step took 4.4 us
+// and a launch gap.
+constexpr int kArgCoef = 64;
+struct Coefs {
+  double c[kArgCoef];
+};
+__device__ __forceinline__ void residual(double* __restrict__ r, const double* __restrict__ V,
+                                         const double* __restrict__ HV, int64_t ldv, const double* c, int m, int64_t n) {
   const double th = c[m];
   for (int64_t i = (int64_t)blockIdx.x * RT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RT) {
     double su = 0, sh = 0;
+#pragma unroll 8
     for (int j = 0; j < m; ++j) {
       su += c[j] * V[(int64_t)j * ldv + i];
       sh += c[j] * HV[(int64_t)j * ldv + i];
     }
-    u[i] = su;
     r[i] = sh - th * su;
   }
+}
+__global__ __launch_bounds__(RT) void k_combine_res(double* __restrict__ r, const double* __restrict__ V,
+                                                     const double* __restrict__ HV, int64_t ldv,
+                                                     const double* __restrict__ c, int m, int64_t n) {
+  residual(r, V, HV, ldv, c, m, n);
+}
+__global__ __launch_bounds__(RT) void k_combine_res_arg(double* __restrict__ r, const double* __restrict__ V,
+                                                         const double* __restrict__ HV, int64_t ldv, Coefs c, int m,
+                                                         int64_t n) {
+  residual(r, V, HV, ldv, c.c, m, n);
 }
 
 // One Gram-Schmidt step fused with the next reduction: w -= sum_j c[j] V_j
@@ -181,8 +194,7 @@ __global__ __launch_bounds__(RT) void k_gs_update_mdot(double* __restrict__ w, c
     }
 #pragma unroll
     for (int q = 0; q < kDotGroup; ++q) {
-      double s = acc[q];
-      for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+      const double s = wave_sum(acc[q]);
       if (lane == 0) red[wv][q] = s;
     }
     __syncthreads();
@@ -200,20 +212,23 @@ __global__ __launch_bounds__(RT) void k_gs_update_mdot(double* __restrict__ w, c
 // / beta with beta^2 = |w|^2 - sum_j c[j]^2, the squared norm of the update
 // for orthonormal V_j.  After a first pass the c[j] are at rounding level
 // relative to |w| and the difference is exact to rounding; when they are
-// not (|c|^2 > |w|^2 / 2: w is rounding noise inside span V, a breakdown)
-// beta = 0 and dst = 0.  Every block sums the partials and the squares in
-// the same order.
+// not (|c|^2 > lim |w|^2) dst = 0 and beta = brk: 0 with lim = 1/2 after a
+// second pass (w is rounding noise inside span V, a breakdown), -1 with a
+// smaller lim where this is the only full pass (w had components in span V
+// after all, and one pass leaves more than rounding of them).  Every block sums
+// the partials and the squares in the same order.
 __global__ __launch_bounds__(RT) void k_gs_update_normalize(const double* __restrict__ w,
                                                              const double* __restrict__ V, int64_t ldv,
                                                              const double* __restrict__ pin, int m, int64_t n,
-                                                             double* __restrict__ dst, double* __restrict__ beta) {
+                                                             double* __restrict__ dst, double* __restrict__ beta,
+                                                             double lim, double brk) {
   __shared__ double c[kMaxM + 1];
   __shared__ double inv;
   sum_coefficients(pin, m + 1, c);
   if (threadIdx.x == 0) {
     double cs = 0;
     for (int j = 0; j < m; ++j) cs += c[j] * c[j];
-    const double b = cs <= 0.5 * c[m] ? sqrt(c[m] - cs) : 0.0;
+    const double b = cs <= lim * c[m] ? sqrt(c[m] - cs) : brk;
     inv = b > 0 ? 1.0 / b : 0.0;
     if (blockIdx.x == 0 && beta) *beta = b;
   }
@@ -263,13 +278,58 @@ __global__ __launch_bounds__(RT) void k_gs_update_mdot_reg(double* __restrict__ 
 #pragma unroll
   for (int q = 0; q <= MC; ++q) {
     if (q < m || (q == MC && wnorm)) {
-      const double t = wave_reduce(acc[q]);
+      const double t = wave_sum(acc[q]);
       if (lane == 0) red[wv][q] = t;
     }
   }
   __syncthreads();
   const int nv = m + (wnorm ? 1 : 0);
   if (threadIdx.x < nv) {
+    const int q = threadIdx.x < m ? threadIdx.x : MC;
+    double t = 0;
+    for (int k = 0; k < RT / 64; ++k) t += red[k][q];
+    pout[(int64_t)threadIdx.x * DOT_BLOCKS + b] = t;
+  }
+}
+
+// Lanczos' first pass: w -= the u <= 2 last vectors U times their coefficients
+// (from the partials pin), then the partials of <V_j, w> (j < m <= MC) and of
+// <w, w>; block 0 writes the last coefficient to cout.  Slices, orders and grid
+// as in k_gs_update_mdot_reg; V's elements are used once, so only the sums stay
+// in registers.  Bound by latency at N = 5e4 (one workgroup per CU, one read of
+// V): 5.0 / 7.6 / 10.3 us for up to 8 / 16 / 32 vectors, where the full first
+// pass (k_mdot_partial over all of V, 4.7 us, and k_gs_update_mdot_reg) took
+// 6.1 / 9.3 / 12.7 us beside its dots.
+template <int MC>
+__global__ __launch_bounds__(RT) void k_gs_local_mdot(double* __restrict__ w, const double* __restrict__ U,
+                                                       int64_t ldv, const double* __restrict__ pin, int u, int64_t n,
+                                                       double* __restrict__ cout, const double* __restrict__ V, int m,
+                                                       double* __restrict__ pout) {
+  __shared__ double red[RT / 64][MC + 1];
+  const double c0 = wave_sum_partials(pin), c1 = u > 1 ? wave_sum_partials(pin + DOT_BLOCKS) : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *cout = u > 1 ? c1 : c0;
+  const int b = blockIdx.x;
+  double acc[MC + 1];
+#pragma unroll
+  for (int q = 0; q <= MC; ++q) acc[q] = 0.0;
+  for (int64_t i = (int64_t)b * RT + threadIdx.x; i < n; i += (int64_t)DOT_BLOCKS * RT) {
+    double wi = w[i] - c0 * U[i];
+    if (u > 1) wi -= c1 * U[ldv + i];
+    w[i] = wi;
+#pragma unroll
+    for (int j = 0; j < MC; ++j)
+      if (j < m) acc[j] += V[(int64_t)j * ldv + i] * wi;
+    acc[MC] += wi * wi;
+  }
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+  for (int q = 0; q <= MC; ++q)
+    if (q < m || q == MC) {
+      const double t = wave_sum(acc[q]);
+      if (lane == 0) red[wv][q] = t;
+    }
+  __syncthreads();
+  if (threadIdx.x <= m) {
     const int q = threadIdx.x < m ? threadIdx.x : MC;
     double t = 0;
     for (int k = 0; k < RT / 64; ++k) t += red[k][q];
@@ -303,14 +363,26 @@ int grid_for(int64_t n) { return (int)std::min<int64_t>(2048, std::max<int64_t>(
 void vec_mdot(const double* V, int64_t ldv, int m, const double* w, int64_t n, double* partial, double* out,
               int accumulate, hipStream_t s) {
   if (m <= 0) return;
-  hipLaunchKernelGGL(k_mdot_partial, dim3(DOT_BLOCKS, m), dim3(RT), 0, s, V, ldv, w, n, partial);
+  hipLaunchKernelGGL(k_mdot_partial, dim3(DOT_BLOCKS, m), dim3(RT), 0, s, V, ldv, m, w, n, partial);
   hipLaunchKernelGGL(k_mdot_final, dim3(m), dim3(RT), 0, s, partial, m, out, accumulate);
 }
 
-void vec_mdot_partial(const double* V, int64_t ldv, int m, const double* w, int64_t n, double* partial,
+void vec_mdot_partial(const double* V, int64_t ldv, int m, const double* w, int64_t n, int wnorm, double* partial,
                       hipStream_t s) {
   if (m <= 0) return;
-  hipLaunchKernelGGL(k_mdot_partial, dim3(DOT_BLOCKS, m), dim3(RT), 0, s, V, ldv, w, n, partial);
+  hipLaunchKernelGGL(k_mdot_partial, dim3(DOT_BLOCKS, m + (wnorm ? 1 : 0)), dim3(RT), 0, s, V, ldv, m, w, n, partial);
+}
+
+void vec_gs_local_mdot(double* w, const double* V, int64_t ldv, const double* pin, int u, int m, int64_t n,
+                       double* cout, double* pout, hipStream_t s) {
+  const double* U = V + (int64_t)(m - u) * ldv;
+  if (m > 32) return vec_gs_update_mdot(w, U, ldv, pin, u, n, cout, u - 1, V, m, 1, pout, s);
+  if (m <= 8)
+    hipLaunchKernelGGL(k_gs_local_mdot<8>, dim3(DOT_BLOCKS), dim3(RT), 0, s, w, U, ldv, pin, u, n, cout, V, m, pout);
+  else if (m <= 16)
+    hipLaunchKernelGGL(k_gs_local_mdot<16>, dim3(DOT_BLOCKS), dim3(RT), 0, s, w, U, ldv, pin, u, n, cout, V, m, pout);
+  else
+    hipLaunchKernelGGL(k_gs_local_mdot<32>, dim3(DOT_BLOCKS), dim3(RT), 0, s, w, U, ldv, pin, u, n, cout, V, m, pout);
 }
 
 void vec_gs_update_mdot(double* w, const double* V, int64_t ldv, const double* pin, int m, int64_t n, double* cout,
@@ -335,10 +407,11 @@ void vec_gs_update_mdot(double* w, const double* V, int64_t ldv, const double* p
 }
 
 void vec_gs_update_normalize(const double* w, const double* V, int64_t ldv, const double* pin, int m, int64_t n,
-                             double* dst, double* beta, hipStream_t s) {
+                             double* dst, double* beta, bool only, hipStream_t s) {
   if (m <= 0) return;
   if (m > kMaxM) fail_vec(m);
-  hipLaunchKernelGGL(k_gs_update_normalize, dim3(grid_for(n)), dim3(RT), 0, s, w, V, ldv, pin, m, n, dst, beta);
+  hipLaunchKernelGGL(k_gs_update_normalize, dim3(grid_for(n)), dim3(RT), 0, s, w, V, ldv, pin, m, n, dst, beta,
+                     only ? kOnePassLim : 0.5, only ? -1.0 : 0.0);
 }
 
 void vec_scale_norm_partial(const double* src, const double* w, double* dst, int64_t n, double* partial,
@@ -356,9 +429,16 @@ void vec_combine(double* y, const double* V, int64_t ldv, const double* c, int m
   hipLaunchKernelGGL(k_combine, dim3(grid_for(n)), dim3(RT), 0, s, y, V, ldv, c, m, n, div);
 }
 
-void vec_combine_res(double* u, double* r, const double* V, const double* HV, int64_t ldv, const double* c, int m,
+void vec_combine_res(double* r, const double* V, const double* HV, int64_t ldv, const double* c, double* dc, int m,
                      int64_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_combine_res, dim3(grid_for(n)), dim3(RT), 0, s, u, r, V, HV, ldv, c, m, n);
+  if (m < kArgCoef) {
+    Coefs a{};
+    std::copy(c, c + m + 1, a.c);
+    hipLaunchKernelGGL(k_combine_res_arg, dim3(grid_for(n)), dim3(RT), 0, s, r, V, HV, ldv, a, m, n);
+    return;
+  }
+  QSX_HIP(hipMemcpyAsync(dc, c, sizeof(double) * (m + 1), hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_combine_res, dim3(grid_for(n)), dim3(RT), 0, s, r, V, HV, ldv, dc, m, n);
 }
 
 }  // namespace qsx

@@ -266,6 +266,52 @@ def test_eigensolvers_vs_dense(gpu, kind):
         assert np.sqrt((w * r) @ r) / np.sqrt((w * gs) @ gs) < 1e-8 * max(1.0, abs(e_ref))
 
 
+@pytest.mark.parametrize("hconj,niter", [(1, 8), (1, 33), (1, 70), (0, 9), (0, 20)])
+def test_eigensolvers_vs_numpy_krylov(gpu, hconj, niter):
+    """Ritz values against the same recurrences in numpy (two full
+    Gram-Schmidt passes a step): beyond the register kernels' 32 vectors and
+    the 64 coefficients of a kernel argument, and (hconj = 0) an operator
+    that is not symmetric, where one pass is not enough.  Tolerance: the
+    recurrences agree to rounding (N eps |H|) while the Krylov basis is the
+    same; 1e-9 |H| leaves three digits for its growth along 70 vectors."""
+    HL, psi, HR = gen.heis_hpsi(seed=25, Dstar=150, mu=1.5, sigma=0.5, dmax=12)
+    H = Q.HPsi(HL, psi, HR, hconj=hconj)
+    S = _dense_weighted(H)
+    assert (np.abs(S - S.T).max() < 1e-12 * np.abs(S).max()) == bool(hconj)
+    sw = np.sqrt(H.weights())
+    x0 = np.random.RandomState(2).standard_normal(H.N)
+
+    def ortho(V, r):
+        first = np.array(V) @ r
+        for _ in range(2):
+            r = r - np.array(V).T @ (np.array(V) @ r)
+        return first, r
+
+    V, al, be, ritz = [sw * x0 / np.linalg.norm(sw * x0)], [], [], []
+    for k in range(1, niter + 1):
+        c, r = ortho(V, S @ V[-1])
+        al.append(c[-1])
+        ritz.append(np.linalg.eigvalsh(np.diag(al) + np.diag(be, 1) + np.diag(be, -1))[0])
+        be.append(np.linalg.norm(r))
+        V.append(r / be[-1])
+    tol = 1e-9 * np.linalg.norm(S, 2)
+    assert np.abs(H.lanczos(x0, niter)[1] - ritz).max() < tol
+    V, ritz = V[:1], []
+    M = np.array([[V[0] @ S @ V[0]]])
+    for k in range(1, niter + 1):
+        lam, y = np.linalg.eigh(M)
+        ritz.append(lam[0])
+        A = np.array(V)
+        _, r = ortho(V, S @ (A.T @ y[:, 0]) - lam[0] * (A.T @ y[:, 0]))
+        if np.linalg.norm(r) < 1e-12 * np.linalg.norm(S, 2):
+            ritz += [lam[0]] * (niter - k)
+            break
+        V.append(r / np.linalg.norm(r))
+        col = np.array(V) @ (S @ V[-1])
+        M = np.block([[M, col[:-1, None]], [col[None, :-1], col[-1:, None]]])
+    assert np.abs(H.davidson(x0, niter)[1] - ritz).max() < tol
+
+
 def test_lanczos_invariant_start(gpu):
     """Lanczos started on an exact eigenvector (the highest, positive
     eigenvalue of a small Heisenberg operator): the Krylov space is
