@@ -229,7 +229,7 @@ struct DevFold {
       so.hconj = 0;
       so.fermA = so.fermB = nullptr;
       std::shared_ptr<CtrPlan> P(plan_create(a.t, ia.data(), (int)ia.size(), cA, cur.t, ib.data(), (int)ib.size(),
-                                             cflag, nullptr, 0, &so, true)
+                                             cflag, nullptr, 0, &so, true, kPlanOnce)
                                      .release());
       double* dC = alloc(P->offsOut.back());
       plan_execute(*P, a.d, cur.d, dC, s);

@@ -726,11 +726,45 @@ static void perm_plan_om(PermPlan& pp, int n, int r, const int64_t* dims, const 
   perm_plan_build(pp, n, r + 1, d.data(), offs, offs, p2.data(), nullptr);
 }
 
+static std::vector<WorkTarget> plan_targets(const CtrPlan& P) {
+  std::vector<WorkTarget> targets(P.nT);
+  for (int t = 0; t < P.nT; ++t) targets[t] = WorkTarget{P.tOff[t], P.M[t], P.N[t], P.pseg[t], P.pseg[t + 1]};
+  return targets;
+}
+
+// The decomposition of a new plan, from its MFMAs (16x16 fragments x k-steps of
+// 4; per SIMD of the chip on average) and fragments F.  Little work: small tiles,
+// shared by a workgroup's waves from few MFMAs on, so the longest chain of
+// dependent loads is short; us of an environment step L.A, X.conj(A) (two plans,
+// SU(2)) in 1x1-fragment tiles shared beyond 8 MFMAs / 2x2 beyond 8 / 2x2 beyond
+// 64: 345 MFMAs a plan 8.1 / 9.3 / 12.0, 3.2e3 8.8 / 11.6 / 16.3, 5.0e3 9.5 / 11.7
+// / 16.4, 1.0e4 13.1 / 12.9 / 16.8, 1.4e4 14.5 / 13.1 / 17.2.  (Between 24 and 44
+// a SIMD as in stage 1 of H*psi.)  A plan used once also pays for building its
+// list, about 0.08 us an item: up to 4x4 fragments a tile; environment update of
+// a U(1) MPS (F = 1.0e4, 5.0e4, 5.7e3; whole call) 3.9 ms against 7.3 ms with 2x2
+// tiles, of which the kernels are 0.12 and 0.08 ms.  Sharing changes the order of
+// a tile's sum: against 80-bit sums the environment step's mean relative errors
+// are 1.6e-16 and 2.6e-16 (L.A, X.conj(A)), unshared 2.1e-16 and 3.3e-16 -- whose
+// sequential order FP64 numpy has as well, so that it differs from that less.
+static void default_policy(CtrPlan& P, bool once) {
+  double mfma = 0, frags = 0;
+  for (int t = 0; t < P.nT; ++t) {
+    const double f = (double)((P.M[t] + 15) / 16) * ((P.N[t] + 15) / 16);
+    double steps = 0;
+    for (int64_t p = P.pseg[t]; p < P.pseg[t + 1]; ++p) steps += (P.pairs[p].K + 3) / 4;
+    frags += f;
+    mfma += f * steps;
+  }
+  const double mean = mfma / 1024;
+  P.policy.wave_max = mean < 8 ? 1 : 2;
+  P.policy.group_mfma = mean < 24 ? 8 : mean < 44 ? 32 : 64;
+  if (once && frags > 4096) P.policy.wave_max = 4;
+}
+
 void plan_upload(CtrPlan& P) {
   PhaseClock clk{P.verbose, "contract plan upload"};
   hipStream_t s = default_stream();
-  std::vector<WorkTarget> targets(P.nT);
-  for (int t = 0; t < P.nT; ++t) targets[t] = WorkTarget{P.tOff[t], P.M[t], P.N[t], P.pseg[t], P.pseg[t + 1]};
+  const std::vector<WorkTarget> targets = plan_targets(P);
   P.work = build_work(targets, P.pairs, P.policy);
   clk.lap("build_work");
   for (void** q : {(void**)&P.dpairs, (void**)&P.ditems, (void**)&P.dreds, (void**)&P.dqueues, (void**)&P.dscratch}) {
@@ -793,7 +827,7 @@ std::unique_ptr<CtrPlan> plan_create(const qsx_tensor* A, const int32_t* ia, int
                                      const qsx_opts* o, bool upload, int force) {
   ensure_device();
   auto P = std::make_unique<CtrPlan>();
-  P->force_layout = force;
+  P->force_layout = force & 3;
   P->A = make_desc(A, "A");
   P->B = make_desc(B, "B");
   if (!ia || !ib || na <= 0 || nb <= 0) fail(QSX_ERR_ARG, "empty contraction index");
@@ -812,6 +846,7 @@ std::unique_ptr<CtrPlan> plan_create(const qsx_tensor* A, const int32_t* ia, int
     fail(QSX_ERR_UNSUPPORTED, "split precision is available for H*psi plans only (QSX_MODE_SPLIT_BF16)");
   build_structure(*P, perm, nperm, o ? o->fermA : nullptr, o ? o->fermB : nullptr);
   PhaseClock clk{P->verbose, "contract plan"};
+  default_policy(*P, force & kPlanOnce);
   if (upload) plan_upload(*P);
   clk.lap("work list + upload");
   return P;
@@ -1018,7 +1053,7 @@ static qsx_tensor_out* contract_oneshot_complex(const qsx_tensor* A, const int32
                                                 const qsx_tensor* B, const int32_t* ib, int nb, int conjB,
                                                 const int32_t* perm, int nperm, const qsx_opts* o) {
   hipStream_t s = default_stream();
-  auto P = plan_create(A, ia, na, conjA, B, ib, nb, conjB, perm, nperm, o, true);
+  auto P = plan_create(A, ia, na, conjA, B, ib, nb, conjB, perm, nperm, o, true, kPlanOnce);
   const bool ai = P->A.hdata_im != nullptr, bi = P->B.hdata_im != nullptr;
   // the plan may have applied the missing-conj rule (contract_getIdxSet)
   const double sA = P->conjA ? -1.0 : 1.0, sB = P->conjB ? -1.0 : 1.0;
@@ -1128,7 +1163,7 @@ qsx_tensor_out* contract_oneshot(const qsx_tensor* A, const int32_t* ia, int na,
   if (A && B && (A->data_im || B->data_im))
     return contract_oneshot_complex(A, ia, na, conjA, B, ib, nb, conjB, perm, nperm, o);
   PhaseClock clk{o ? o->verbose : 0, "contract"};
-  auto P = plan_create(A, ia, na, conjA, B, ib, nb, conjB, perm, nperm, o, true);
+  auto P = plan_create(A, ia, na, conjA, B, ib, nb, conjB, perm, nperm, o, true, kPlanOnce);
   clk.lap("plan (structure + upload)");
   double *dA = (double*)dev_alloc(sizeof(double) * std::max<int64_t>(1, P->A.total()));
   double *dB = (double*)dev_alloc(sizeof(double) * std::max<int64_t>(1, P->B.total()));
