@@ -23,11 +23,15 @@
 // leaves a relative error of about 2^{-7S} of |row| |col| per term: S = 6
 // gives ~1e-13 relative to the operand scale; S <= 5 does not reach 1e-12.
 //
-// Layout: each contraction line is stored packed, quads of 4 consecutive k
-// with the S slices of each quad together (slice s of element k at
-// pbase + (k/4) 4S + 4s + k%4; the tail of the last quad is zero), so a lane
-// loads the slices of its row (column) and quad of k as S 8-byte runs;
-// exponents are int32 per line.  One wave computes one 16x16 output tile
+// Layout: the lines of an operand block in groups of 16, k in blocks of 16, the S
+// slices of a (group, k block) one after the other, each slice as its 64 quads
+// of 4 consecutive k in the MFMA's lane order (quad (k%16)/4 of line l%16 at
+// place 16 (k%16)/4 + l%16), zero beyond the block: one slice of an operand
+// fragment is one contiguous load of the wave (512 bytes; 1 KB in FP32).
+// (Each line's own quads in a row instead, 56 bytes per quad, scattered every
+// load over 64 cache lines and every store over as many: 36.8 us per GEMM at
+// D* = 4000, 20.7 us now, with the next k block's loads behind the MFMAs.)  Exponents are int32
+// per line.  One wave computes one 16x16 output tile
 // (v_mfma_f32_16x16x16bf16_1k: A lane l holds row l%16, k 4(l/16)..+3;
 // B lane l holds k 4(l/16)..+3, col l%16; result element v of lane l is
 // row 4(l/16)+v, col l%16 -- checked on the device with exact integers), or
@@ -47,46 +51,73 @@ typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int NT = 256;
-constexpr int kBits = 7;       // bits per slice
 constexpr int kFlushK = 128;   // k per exact FP32 accumulation window
 constexpr int kSlot = 64 * 64; // scratch doubles per partial tile (the wave engine's reduce reads them)
+constexpr int kGroupElems = kSplitGroupElems;
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
-// position of slice s of element k of a line in its packed storage: quads of
-// 4 consecutive k, each quad holding its S slices of 4 values
-__device__ __forceinline__ int64_t packed_at(const SplitLine& L, int k, int s, int S) {
-  return L.pbase + (int64_t)(k >> 2) * (4 * S) + 4 * s + (k & 3);
+// position of slice s of quad q of a line (pbase: its place in its group's
+// first k block)
+__device__ __forceinline__ int64_t packed_at(const SplitLine& L, int q, int s, int S) {
+  return L.pbase + ((int64_t)(q >> 2) * S + s) * kGroupElems + (q & 3) * 64;
 }
 
-// BF16 slices of one element (7 bits each, exact in BF16)
-__device__ __forceinline__ void slice_bf16(double x, int e, int S, const SplitLine& L, int k,
-                                           uint16_t* __restrict__ P) {
-  double r = ldexp(x, -e);
-  for (int s = 0; s < S; ++s) {
-    const double q = rint(ldexp(r, kBits * (s + 1)));
-    const double sig = ldexp(q, -kBits * (s + 1));
-    r -= sig;
-    // sig has at most 8 significant bits: exact in FP32 and in BF16
-    P[packed_at(L, k, s, S)] = (uint16_t)(__float_as_uint((float)sig) >> 16);
+// the slices of a quad of elements, scaled by 2^-e.  BF16: with t_s = r_s 2^(7s),
+// q_s = rint(128 t_s), t_{s+1} = 128 t_s - q_s (exact) and sigma_s = q_s 2^-7(s+1)
+// (at most 8 significant bits, exact in FP32 and BF16).  FP32 x 3: sigma_0 on
+// the 2^-11 grid, sigma_1 and sigma_2 the FP32 roundings of the remainders.
+template <typename T, bool F32>
+__device__ __forceinline__ void slice_quad(const double (&x)[4], int e, int S, const SplitLine& L, int q,
+                                           T* __restrict__ P) {
+  if constexpr (F32) {
+    f4 o[3];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      double r = ldexp(x[j], -e);
+      const double s0 = rint(r * 2048.0) * (1.0 / 2048.0);
+      r -= s0;
+      const float s1 = (float)r;
+      r -= (double)s1;
+      o[0][j] = (float)s0;
+      o[1][j] = s1;
+      o[2][j] = (float)r;
+    }
+#pragma unroll
+    for (int s = 0; s < 3; ++s) *(f4*)((float*)P + packed_at(L, q, s, 3)) = o[s];
+  } else {
+    double t[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) t[j] = ldexp(x[j], -e);
+    float scale = 1.0f;
+    for (int s = 0; s < S; ++s) {
+      scale *= 1.0f / 128.0f;
+      s4 o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const double u = t[j] * 128.0, n = rint(u);
+        t[j] = u - n;
+        o[j] = (short)(__float_as_uint((float)n * scale) >> 16);
+      }
+      *(s4*)((uint16_t*)P + packed_at(L, q, s, S)) = o;
+    }
   }
 }
 
-// FP32 x 3 slices of one element: sigma_0 on the 2^-11 grid, sigma_1 and
-// sigma_2 the FP32 roundings of the remainders
-__device__ __forceinline__ void slice_f32(double x, int e, const SplitLine& L, int k, float* __restrict__ P) {
-  double r = ldexp(x, -e);
-  const double s0 = ldexp(rint(ldexp(r, 11)), -11);
-  r -= s0;
-  const float s1 = (float)r;
-  r -= (double)s1;
-  P[packed_at(L, k, 0, 3)] = (float)s0;
-  P[packed_at(L, k, 1, 3)] = s1;
-  P[packed_at(L, k, 2, 3)] = (float)r;
+__device__ __forceinline__ void load_quad(const SplitLine& L, const double* __restrict__ X, int q, double (&x)[4]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int k = 4 * q + j;
+    x[j] = k < L.K ? X[L.off + (int64_t)k * L.sk] : 0.0;
+  }
 }
 
-// one wave per contraction line (lines contiguous along k): exponent, then
-// the slices of each element
+__device__ __forceinline__ double quad_max(const double (&x)[4]) {
+  return fmax(fmax(fabs(x[0]), fabs(x[1])), fmax(fabs(x[2]), fabs(x[3])));
+}
+
+// one wave per contraction line (lines contiguous along k), a quad per lane:
+// exponent (max |x| < 2^e), then the slices
 template <typename T, bool F32>
 __global__ __launch_bounds__(NT) void k_split_lines(const SplitLine* __restrict__ lines, int nlines,
                                                     const double* __restrict__ X, T* __restrict__ P, int S,
@@ -95,112 +126,64 @@ __global__ __launch_bounds__(NT) void k_split_lines(const SplitLine* __restrict_
   if (li >= nlines) return;
   const int lane = threadIdx.x & 63;
   const SplitLine L = lines[li];
-  double mx = 0.0;
-  for (int k = lane; k < L.K; k += 64) mx = fmax(mx, fabs(X[L.off + (int64_t)k * L.sk]));
+  const int nq = (L.K + 3) >> 2;
+  double x[4] = {0.0, 0.0, 0.0, 0.0}, mx = 0.0;
+  for (int q = lane; q < nq; q += 64) {
+    load_quad(L, X, q, x);
+    mx = fmax(mx, quad_max(x));
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-  // max |x| < 2^e
   const int e = mx > 0.0 ? ilogb(mx) + 1 : 0;
   if (lane == 0) exps[L.eidx] = e;
-  for (int k = lane; k < L.K; k += 64) {
-    const double x = X[L.off + (int64_t)k * L.sk];
-    if constexpr (F32) slice_f32(x, e, L, k, (float*)P);
-    else slice_bf16(x, e, S, L, k, (uint16_t*)P);
+  for (int q = lane; q < nq; q += 64) {
+    if (nq > 64) load_quad(L, X, q, x);
+    slice_quad<T, F32>(x, e, S, L, q, P);
   }
 }
 
-// Lines whose elements are strided while neighbouring lines are adjacent
-// (e.g. the rows of a column-major block) run in two passes over a 2-D grid
-// of (16 lines, 64 k) waves, 4 lanes per line, so that each load instruction
-// reads 16 adjacent elements: the exponents (chunk maxima merged by an
-// integer maximum), then the slices, each lane writing a quad's slices as
-// one run.
-constexpr int kQuadsPerWave = 16;  // quads of 4 k per wave of both passes
-constexpr int kNoExp = -100000;    // exponent of a line not yet seen non-zero
-
-__global__ __launch_bounds__(NT) void k_exps_fill(int32_t* __restrict__ exps, int n) {
-  const int i = blockIdx.x * NT + threadIdx.x;
-  if (i < n) exps[i] = kNoExp;
-}
-
-// per (16 lines, chunk of k) wave: the chunk's maximum of each line, its
-// exponent merged into the line's by an integer maximum (the exponent is
-// monotonic in the maximum)
-__global__ __launch_bounds__(NT) void k_split_exps_grp(const SplitLine* __restrict__ lines, int nlines,
-                                                       const double* __restrict__ X, int32_t* __restrict__ exps) {
-  const int lane = threadIdx.x & 63;
-  const int li = (blockIdx.x * (NT / 64) + (threadIdx.x >> 6)) * 16 + (lane & 15), kq = lane >> 4;
-  const bool ok = li < nlines;
+// lines whose elements are strided while neighbouring lines are adjacent (e.g.
+// the rows of a column-major block): one workgroup per 16 lines, lane l taking
+// line l%16 and every 16th quad, so that each load reads 16 adjacent elements
+// and each store 16 adjacent quads; the waves' maxima meet in LDS.  A lane's
+// first two quads stay in registers between the maximum and the slices (k <=
+// 128: one read).  One launch where the exponents took a fill, an integer
+// atomic maximum over a 2-D grid and a second read (three launches, 3.4 + 8.7 +
+// 22 us at D* = 4000, intermediate and operators; 23 us now).  Whole H*psi with
+// 7 slices, D* = 4000: 136 -> 90 us.
+template <typename T, bool F32>
+__global__ __launch_bounds__(NT) void k_split_groups(const SplitLine* __restrict__ lines, int nlines,
+                                                     const double* __restrict__ X, T* __restrict__ P, int S,
+                                                     int32_t* __restrict__ exps) {
+  constexpr int NQ = NT / 16;  // quads per round
+  __shared__ double wm[NT / 64][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int li = blockIdx.x * 16 + (lane & 15), q0 = wave * 4 + (lane >> 4);
   SplitLine L{};
-  if (ok) L = lines[li];
-  double mx = 0.0;
-  if (ok) {
-    const int nq = (L.K + 3) >> 2, q1 = min(nq, (int)(blockIdx.y + 1) * kQuadsPerWave);
-    for (int q = (int)blockIdx.y * kQuadsPerWave + kq; q < q1; q += 4) {
-      double x[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int k = 4 * q + j;
-        x[j] = k < L.K ? fabs(X[L.off + (int64_t)k * L.sk]) : 0.0;
-      }
-      mx = fmax(mx, fmax(fmax(x[0], x[1]), fmax(x[2], x[3])));
-    }
+  if (li < nlines) L = lines[li];
+  const int nq = (L.K + 3) >> 2;
+  double x[4], y[4];
+  load_quad(L, X, q0, x);
+  load_quad(L, X, q0 + NQ, y);
+  double mx = fmax(quad_max(x), quad_max(y));
+  for (int q = q0 + 2 * NQ; q < nq; q += NQ) {
+    double z[4];
+    load_quad(L, X, q, z);
+    mx = fmax(mx, quad_max(z));
   }
   mx = fmax(mx, __shfl_xor(mx, 16, 64));
   mx = fmax(mx, __shfl_xor(mx, 32, 64));
-  if (ok && kq == 0 && mx > 0.0) atomicMax(exps + L.eidx, ilogb(mx) + 1);
-}
-
-template <typename T, bool F32>
-__global__ __launch_bounds__(NT) void k_split_quads_grp(const SplitLine* __restrict__ lines, int nlines,
-                                                        const double* __restrict__ X, T* __restrict__ P, int S,
-                                                        const int32_t* __restrict__ exps) {
-  const int lane = threadIdx.x & 63;
-  const int li = (blockIdx.x * (NT / 64) + (threadIdx.x >> 6)) * 16 + (lane & 15), kq = lane >> 4;
-  if (li >= nlines) return;
-  const SplitLine L = lines[li];
-  const int e = exps[L.eidx] == kNoExp ? 0 : exps[L.eidx];
-  const int nq = (L.K + 3) >> 2, q1 = min(nq, (int)(blockIdx.y + 1) * kQuadsPerWave);
-  for (int q = (int)blockIdx.y * kQuadsPerWave + kq; q < q1; q += 4) {
-    double x[4];
+  if (lane < 16) wm[wave][lane] = mx;
+  __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = 4 * q + j;
-      x[j] = k < L.K ? X[L.off + (int64_t)k * L.sk] : 0.0;
-    }
-    if constexpr (F32) {
-      f4 o0, o1, o2;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        double r = ldexp(x[j], -e);
-        const double s0 = ldexp(rint(ldexp(r, 11)), -11);
-        r -= s0;
-        const float s1 = (float)r;
-        r -= (double)s1;
-        o0[j] = (float)s0;
-        o1[j] = s1;
-        o2[j] = (float)r;
-      }
-      f4* d = (f4*)((float*)P + L.pbase + (int64_t)q * 12);
-      d[0] = o0;
-      d[1] = o1;
-      d[2] = o2;
-    } else {
-      double r[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) r[j] = ldexp(x[j], -e);
-      s4* d = (s4*)((uint16_t*)P + L.pbase + (int64_t)q * 4 * S);
-      for (int s = 0; s < S; ++s) {
-        s4 o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const double sig = ldexp(rint(ldexp(r[j], kBits * (s + 1))), -kBits * (s + 1));
-          r[j] -= sig;
-          o[j] = (short)(__float_as_uint((float)sig) >> 16);
-        }
-        d[s] = o;
-      }
-    }
+  for (int w = 0; w < NT / 64; ++w) mx = fmax(mx, wm[w][lane & 15]);
+  const int e = mx > 0.0 ? ilogb(mx) + 1 : 0;
+  if (threadIdx.x < 16 && li < nlines) exps[L.eidx] = e;
+  if (q0 < nq) slice_quad<T, F32>(x, e, S, L, q0, P);
+  if (q0 + NQ < nq) slice_quad<T, F32>(y, e, S, L, q0 + NQ, P);
+  for (int q = q0 + 2 * NQ; q < nq; q += NQ) {
+    load_quad(L, X, q, x);
+    slice_quad<T, F32>(x, e, S, L, q, P);
   }
 }
 
@@ -226,10 +209,22 @@ __device__ __forceinline__ void store_tile(const WorkItem& w, const double (&c64
   }
 }
 
-// BF16 slices: per k-step of 16 each lane loads, for its row of A (its
-// column of B) and its quad of 4 k, the S slices as S 8-byte runs of the
-// packed line (v_mfma_f32_16x16x16bf16_1k: A lane l holds row l%16, k
-// 4(l/16)..+3; B lane l holds k 4(l/16)..+3, column l%16)
+// The lanes' quads of the k block at k that lie in the chunk [kb, ke) of a pair
+// of depth K; every other quad of the block is zeroed (the padding beyond K
+// is stored as zeros)
+template <int S, typename V>
+__device__ __forceinline__ void mask_chunk(V (&a)[S], int k, int kb, int ke, int K) {
+  if (k >= kb && (k + 16 <= ke || ke == K)) return;  // uniform
+  const int kq = k + 4 * ((threadIdx.x & 63) >> 4);
+  if (kq >= kb && kq < ke) return;
+#pragma unroll
+  for (int s = 0; s < S; ++s) a[s] = V{0, 0, 0, 0};
+}
+
+// BF16 slices: per k block of 16 a lane's 8 bytes of every slice of both
+// fragments (v_mfma_f32_16x16x16bf16_1k: A lane l holds row l%16, k
+// 4(l/16)..+3; B lane l holds k 4(l/16)..+3, column l%16); the next block's are
+// in flight behind the MFMAs
 template <int S>
 __global__ __launch_bounds__(NT) void k_split_gemm(const WorkItem* __restrict__ items, int nitems,
                                                    const SplitPair* __restrict__ pairs,
@@ -241,15 +236,26 @@ __global__ __launch_bounds__(NT) void k_split_gemm(const WorkItem* __restrict__ 
   const WorkItem w = items[wid];
   if (w.slot == -2) return;
   const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
-  const int row = w.m0 + lr, col = w.n0 + lr;
-  const bool rowok = row < w.M, colok = col < w.N;
+  const int col = w.n0 + lr;
+  const bool colok = col < w.N;
   double c64[4] = {0.0, 0.0, 0.0, 0.0};
   for (int p = w.p0; p <= w.p1; ++p) {
     const SplitPair pd = pairs[p];
     const int kb = p == w.p0 ? w.k0 : 0, ke = p == w.p1 ? w.k1 : pd.K;
-    const int64_t lenq = (int64_t)((pd.K + 3) >> 2) * (4 * S);  // packed length of a line
-    const s4* pa = (const s4*)(Ap + pd.pa + (int64_t)(rowok ? row : 0) * lenq);
-    const s4* pb = (const s4*)(Bp + pd.pb + (int64_t)(colok ? col : 0) * lenq);
+    const int64_t grp = (int64_t)((pd.K + 15) >> 4) * (S * kGroupElems);  // a group of 16 lines
+    const s4* pa = (const s4*)(Ap + pd.pa + (w.m0 >> 4) * grp) + lane;
+    const s4* pb = (const s4*)(Bp + pd.pb + (w.n0 >> 4) * grp) + lane;
+    const int kf = kb & ~15;
+    s4 a[S], b[S], an[S], bn[S];
+    auto fetch = [&](int k, s4(&u)[S], s4(&v)[S]) {
+      const int o = (k >> 4) * (S * kGroupElems / 4);
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        u[s] = pa[o + s * (kGroupElems / 4)];
+        v[s] = pb[o + s * (kGroupElems / 4)];
+      }
+    };
+    if (kf < ke) fetch(kf, a, b);
     int er[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -261,16 +267,9 @@ __global__ __launch_bounds__(NT) void k_split_gemm(const WorkItem* __restrict__ 
 #pragma unroll
     for (int u = 0; u < S; ++u) acc[u] = f4{0.f, 0.f, 0.f, 0.f};
     int win = 0;
-    for (int k = kb; k < ke; k += 16) {
-      const int kq = k + 4 * lq;
-      const bool in = kq < ke;
-      const int q = kq >> 2;
-      s4 a[S], b[S];
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        a[s] = in && rowok ? pa[(int64_t)q * S + s] : s4{0, 0, 0, 0};
-        b[s] = in && colok ? pb[(int64_t)q * S + s] : s4{0, 0, 0, 0};
-      }
+    for (int k = kf; k < ke; k += 16) {
+      if (k + 16 < ke) fetch(k + 16, an, bn);
+      mask_chunk<S>(a, k, kb, ke, pd.K);  // a zero operand suffices
 #pragma unroll
       for (int u = 0; u < S; ++u)
 #pragma unroll
@@ -288,6 +287,11 @@ __global__ __launch_bounds__(NT) void k_split_gemm(const WorkItem* __restrict__ 
 #pragma unroll
         for (int u = 0; u < S; ++u) acc[u] = f4{0.f, 0.f, 0.f, 0.f};
         win = 0;
+      }
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        a[s] = an[s];
+        b[s] = bn[s];
       }
     }
   }
@@ -315,7 +319,7 @@ __global__ __launch_bounds__(NT) void k_split_gemm(const WorkItem* __restrict__ 
 // Per k-step of 16 lane group g takes the quad k + 4g..+3 for the 4 MFMAs
 // (MFMA j uses element j of every group's quad: the k order inside the step
 // is permuted, which the sum does not see), so each lane loads its 3 slices
-// as 3 16-byte runs of the packed line.
+// as 16 bytes of 3 contiguous 1 KB runs.
 constexpr int kF32Win = 32;  // k per FP32 accumulation window of u = 1, 2
 
 __global__ __launch_bounds__(NT) void k_split_gemm_f32(const WorkItem* __restrict__ items, int nitems,
@@ -328,15 +332,15 @@ __global__ __launch_bounds__(NT) void k_split_gemm_f32(const WorkItem* __restric
   const WorkItem w = items[wid];
   if (w.slot == -2) return;
   const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
-  const int row = w.m0 + lr, col = w.n0 + lr;
-  const bool rowok = row < w.M, colok = col < w.N;
+  const int col = w.n0 + lr;
+  const bool colok = col < w.N;
   double c64[4] = {0.0, 0.0, 0.0, 0.0};
   for (int p = w.p0; p <= w.p1; ++p) {
     const SplitPair pd = pairs[p];
     const int kb = p == w.p0 ? w.k0 : 0, ke = p == w.p1 ? w.k1 : pd.K;
-    const int64_t lenq = (int64_t)((pd.K + 3) >> 2) * 12;
-    const f4* pa = (const f4*)(Ap + pd.pa + (int64_t)(rowok ? row : 0) * lenq);
-    const f4* pb = (const f4*)(Bp + pd.pb + (int64_t)(colok ? col : 0) * lenq);
+    const int64_t grp = (int64_t)((pd.K + 15) >> 4) * (3 * kGroupElems);  // a group of 16 lines
+    const f4* pa = (const f4*)(Ap + pd.pa + (w.m0 >> 4) * grp) + lane;
+    const f4* pb = (const f4*)(Bp + pd.pb + (w.n0 >> 4) * grp) + lane;
     double sc[4];
     const int fc = colok ? expB[pd.eb + col] : 0;
 #pragma unroll
@@ -346,15 +350,22 @@ __global__ __launch_bounds__(NT) void k_split_gemm_f32(const WorkItem* __restric
     }
     f4 acc1 = f4{0.f, 0.f, 0.f, 0.f}, acc2 = f4{0.f, 0.f, 0.f, 0.f};
     int win = 0;
-    for (int k = kb; k < ke; k += 16) {
-      const int kq = k + 4 * lq;
-      const bool in = kq < ke;
-      const int64_t q = kq >> 2;
-      const f4 z = f4{0.f, 0.f, 0.f, 0.f};
-      const f4 a0 = in && rowok ? pa[q * 3] : z, a1 = in && rowok ? pa[q * 3 + 1] : z,
-               a2 = in && rowok ? pa[q * 3 + 2] : z;
-      const f4 b0 = in && colok ? pb[q * 3] : z, b1 = in && colok ? pb[q * 3 + 1] : z,
-               b2 = in && colok ? pb[q * 3 + 2] : z;
+    const f4 z = f4{0.f, 0.f, 0.f, 0.f};
+    const int kf = kb & ~15;
+    f4 a[3] = {z, z, z}, b[3] = {z, z, z}, an[3], bn[3];
+    auto fetch = [&](int k, f4(&u)[3], f4(&v)[3]) {
+      const int o = (k >> 4) * (3 * kGroupElems / 4);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        u[s] = pa[o + s * (kGroupElems / 4)];
+        v[s] = pb[o + s * (kGroupElems / 4)];
+      }
+    };
+    if (kf < ke) fetch(kf, a, b);
+    for (int k = kf; k < ke; k += 16) {
+      if (k + 16 < ke) fetch(k + 16, an, bn);
+      mask_chunk<3>(a, k, kb, ke, pd.K);  // a zero operand suffices
+      const f4 a0 = a[0], a1 = a[1], a2 = a[2], b0 = b[0], b1 = b[1], b2 = b[2];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const f4 acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[j], b0[j], z, 0, 0, 0);
@@ -374,23 +385,23 @@ __global__ __launch_bounds__(NT) void k_split_gemm_f32(const WorkItem* __restric
         acc2 = z;
         win = 0;
       }
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        a[s] = an[s];
+        b[s] = bn[s];
+      }
     }
   }
   store_tile(w, c64, C, scratch);
 }
 
 template <typename T, bool F32>
-void lines_launch(const SplitLine* dlines, int nlines, int maxk, bool grouped, const double* X, T* P, int S,
+void lines_launch(const SplitLine* dlines, int nlines, bool grouped, const double* X, T* P, int S,
                   int32_t* exps, hipStream_t s) {
   if (nlines <= 0) return;
   if (grouped) {
-    const int nb = (nlines + 16 * (NT / 64) - 1) / (16 * (NT / 64));
-    const int ny = std::max(1, ((maxk + 3) / 4 + kQuadsPerWave - 1) / kQuadsPerWave);
-    // line indices are the exponent indices 0 .. nlines-1
-    hipLaunchKernelGGL(k_exps_fill, dim3((nlines + NT - 1) / NT), dim3(NT), 0, s, exps, nlines);
-    hipLaunchKernelGGL(k_split_exps_grp, dim3(nb, ny), dim3(NT), 0, s, dlines, nlines, X, exps);
-    QSX_HIP(hipGetLastError());
-    hipLaunchKernelGGL((k_split_quads_grp<T, F32>), dim3(nb, ny), dim3(NT), 0, s, dlines, nlines, X, P, S, exps);
+    hipLaunchKernelGGL((k_split_groups<T, F32>), dim3((nlines + 15) / 16), dim3(NT), 0, s, dlines, nlines, X, P, S,
+                       exps);
   } else {
     const int nb = (nlines + NT / 64 - 1) / (NT / 64);
     hipLaunchKernelGGL((k_split_lines<T, F32>), dim3(nb), dim3(NT), 0, s, dlines, nlines, X, P, S, exps);
@@ -400,14 +411,14 @@ void lines_launch(const SplitLine* dlines, int nlines, int maxk, bool grouped, c
 
 }  // namespace
 
-void launch_split_lines(const SplitLine* dlines, int nlines, int maxk, bool per_lane, const double* X,
+void launch_split_lines(const SplitLine* dlines, int nlines, bool per_lane, const double* X,
                         uint16_t* planes, int S, int32_t* exps, hipStream_t s) {
-  lines_launch<uint16_t, false>(dlines, nlines, maxk, per_lane, X, planes, S, exps, s);
+  lines_launch<uint16_t, false>(dlines, nlines, per_lane, X, planes, S, exps, s);
 }
 
-void launch_split_lines_f32(const SplitLine* dlines, int nlines, int maxk, bool per_lane, const double* X,
+void launch_split_lines_f32(const SplitLine* dlines, int nlines, bool per_lane, const double* X,
                             float* planes, int32_t* exps, hipStream_t s) {
-  lines_launch<float, true>(dlines, nlines, maxk, per_lane, X, planes, 3, exps, s);
+  lines_launch<float, true>(dlines, nlines, per_lane, X, planes, 3, exps, s);
 }
 
 void launch_split_gemm(int S, const WorkItem* ditems, int nitems, const SplitPair* dpairs, const uint16_t* Ap,

@@ -375,6 +375,27 @@ def test_split_precision_slices(gpu):
     assert errs[3] > 1e-9, errs  # the slices really are narrow
 
 
+@pytest.mark.parametrize("kw", [dict(Dstar=40, mu=1.2, sigma=0.4, dmax=6), dict(Dstar=300, mu=3.5, sigma=0.3, dmax=40),
+                                dict(Dstar=700, mu=5.0, sigma=0.25, dmax=300),
+                                dict(Dstar=900, mu=5.6, sigma=0.1, dmax=400)])
+def test_split_block_sizes(gpu, kw):
+    """both split modes over block sizes that cross the packed layout's edges
+    (blocks of 2..6 states; around 16 and 32; k beyond the 128 and 256 that
+    the slicing keeps in registers and the accumulation flushes at, with
+    k-ranges cut inside a block of 16), with zero rows and columns; against
+    the FP64 plan, to the modes' stated bounds (1e-12, 5e-10)"""
+    HL, psi, HR = gen.heis_hpsi(seed=31, **kw)
+    data = [d.copy() for d in HL.data]
+    data[0][0] = 0.0
+    data[-1][:, -1] = 0.0
+    HL = HL.with_packed(np.concatenate([d.ravel(order="F") for d in data]))
+    x = np.random.RandomState(3).standard_normal(psi.numel())
+    ref = Q.HPsi(HL, psi, HR, hconj=1).apply(x)
+    for mode, bound in (("split_bf16", TOL), ("split_f32", 5e-10)):
+        got = Q.HPsi(HL, psi, HR, hconj=1, mode=mode).apply(x)
+        assert np.linalg.norm(got - ref) <= bound * np.linalg.norm(ref), mode
+
+
 def test_split_precision_config4_vs_oracle(gpu, heis4000):
     """config 4 (the headline operator at D* = 4000) in split precision with
     the default slice count: within 1e-12 of the oracle; at full size the
