@@ -66,18 +66,12 @@ __device__ __forceinline__ bool rotate_pair(double* ap, double* aq, double* vp, 
   constexpr int L = SVD_SEG;
   double c, s;
   if constexpr (R > 0) {
-    // V's elements are fetched with A's when registers allow (R <= 4)
-    constexpr bool pre = R <= 4;
     double x[R], y[R], u[R], z[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = lane + L * r;
       x[r] = i < m ? ap[i] : 0.0;
       y[r] = i < m ? aq[i] : 0.0;
-      if (pre) {
-        u[r] = i < n ? vp[i] : 0.0;
-        z[r] = i < n ? vq[i] : 0.0;
-      }
     }
     double al = 0.0, be = 0.0, ga = 0.0;
 #pragma unroll
@@ -98,13 +92,11 @@ __device__ __forceinline__ bool rotate_pair(double* ap, double* aq, double* vp, 
         aq[i] = s * x[r] + c * y[r];
       }
     }
-    if (!pre) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int i = lane + L * r;
-        u[r] = i < n ? vp[i] : 0.0;
-        z[r] = i < n ? vq[i] : 0.0;
-      }
+    for (int r = 0; r < R; ++r) {
+      const int i = lane + L * r;
+      u[r] = i < n ? vp[i] : 0.0;
+      z[r] = i < n ? vq[i] : 0.0;
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
