@@ -249,8 +249,8 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   hipStream_t s = default_stream();
   std::vector<SvdGather> gath;
   std::vector<SvdItem> items;
-  std::vector<SvdGroup> qr;  // the groups reduced by QR; the others in `big`
-  std::vector<int32_t> big;
+  std::vector<SvdGroup> qr;         // the groups reduced by QR
+  std::vector<int32_t> whole, big;  // the others: in one workgroup's LDS, beyond it
   int64_t work = 0, nsig = 0, nperm = 0;
   auto take = [&](int64_t n) {  // buffers start at multiples of 16 doubles
     const int64_t o = work;
@@ -288,7 +288,7 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
       q.c2 = take((int64_t)q.n16 * q.n16);
       qr.push_back(q);
     } else {
-      big.push_back((int32_t)items.size());
+      (b.m * b.n + b.n * b.n <= SVD_LDS_DOUBLES ? whole : big).push_back((int32_t)items.size());
     }
     items.push_back(it);
     for (size_t t = 0; t < b.blk.size(); ++t) {
@@ -412,7 +412,10 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
       for (void* x : p) dev_free(x);
     }
   } fr;
-  // groups beyond the QR's range: block one-sided Jacobi over column blocks
+  for (int32_t i : whole)
+    if ((int64_t)items[i].m * items[i].n + (int64_t)items[i].n * items[i].n > SVD_LDS_DOUBLES)
+      fail(QSX_ERR_STRUCT, "orthoQS: internal SVD item beyond the LDS");
+  // groups beyond the QR's range and the LDS: block one-sided Jacobi over column blocks
   // of at most cb columns, two blocks (and their columns of V) staged in LDS
   // per workgroup
   std::vector<int32_t> nbk, cbk;
@@ -437,6 +440,7 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   };
   SvdItem* ditems = put(items);
   SvdGather* dgath = put(gath);
+  int32_t* dwhole = put(whole);
   int32_t* dbig = put(big);
   SvdGroup* dqr = put(qr);
   SvdQr* dqr1 = put(qr1);
@@ -448,7 +452,7 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   SvdBlockStep* drsteps = put(rsteps);
   int32_t* dperm = (int32_t*)fr.add(sizeof(int32_t) * std::max<int64_t>(1, nperm));
   int32_t* dexpo = (int32_t*)fr.add(sizeof(int32_t) * std::max<size_t>(1, qr.size()));
-  int32_t* dsw = (int32_t*)fr.add(sizeof(int32_t) * std::max<size_t>(1, small.size()));
+  int32_t* dsw = (int32_t*)fr.add(sizeof(int32_t) * std::max<size_t>(1, small.size() + whole.size()));
   const size_t nrot = (size_t)jacobi_max_sweeps() * qr.size();
   int32_t* drot = (int32_t*)fr.add(sizeof(int32_t) * std::max(nrot, items.size()));
   upload_packed(P, P.hdata, dpsi.p, s);
@@ -477,6 +481,7 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   QSX_HIP(hipEventRecord(ready.e, s));
   QSX_HIP(hipStreamWaitEvent(s2, ready.e, 0));
   launch_jacobi_lds(dqr, dsmall, (int)small.size(), dwork.p, dsw, s2);
+  launch_jacobi_whole(ditems, dwhole, (int)whole.size(), dwork.p, dsig.p, dsw + small.size(), s2);
   QSX_HIP(hipEventRecord(done.e, s2));
   int maxsw = 0;
   if (!big.empty()) {
@@ -574,10 +579,10 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   launch_svd_vectors(dqr, (int)qr.size(), maxn, dwork.p, dsig.p, dexpo, s);
   launch_svd_applyq(dapp, (int)app.size(), maxrows, dwork.p, dperm, s);
   std::vector<double> sig(nsig);
-  std::vector<int32_t> sweeps(small.size());
+  std::vector<int32_t> sweeps(small.size() + whole.size());
   QSX_HIP(hipMemcpyAsync(sig.data(), dsig.p, sizeof(double) * nsig, hipMemcpyDeviceToHost, s));
-  if (!small.empty())
-    QSX_HIP(hipMemcpyAsync(sweeps.data(), dsw, sizeof(int32_t) * small.size(), hipMemcpyDeviceToHost, s));
+  if (!sweeps.empty())
+    QSX_HIP(hipMemcpyAsync(sweeps.data(), dsw, sizeof(int32_t) * sweeps.size(), hipMemcpyDeviceToHost, s));
   QSX_HIP(hipStreamSynchronize(s));
   for (int x : sweeps) {
     if (x >= jacobi_max_sweeps()) fail(QSX_ERR_ARG, "orthoQS: Jacobi SVD did not converge in %d sweeps", x);

@@ -400,8 +400,8 @@ void launch_fill_zero(double* p, int64_t n, hipStream_t s);
 // (the transpose of a wide matrix).  Up to SVD_QR_MAX_M x SVD_QR_MAX_N it is
 // reduced to an n x n triangle by QR first and decomposed there, in one
 // workgroup's LDS for n <= SVD_LDS_N and by rounds of column blocks beyond;
-// a larger one is decomposed as it is by column-block steps with
-// SVD_LDS_DOUBLES of LDS.
+// another one is decomposed as it is, in one workgroup's LDS when m n + n^2 <=
+// SVD_LDS_DOUBLES, by column-block steps beyond.
 constexpr int SVD_QR_MAX_M = 1024;
 constexpr int SVD_QR_MAX_N = 256;
 constexpr int SVD_LDS_N = 96;         // 2 n (n + 8) doubles fit a workgroup's LDS
@@ -462,6 +462,8 @@ void launch_svd_applyq(const SvdApply* ditems, int nitems, int maxrows, double* 
 // sweeps[i] = sweeps that rotated (jacobi_max_sweeps(): not converged)
 void launch_jacobi_lds(const SvdGroup* dgroups, const int32_t* dwhich, int n, double* work, int32_t* sweeps,
                        hipStream_t s);
+void launch_jacobi_whole(const SvdItem* ditems, const int32_t* dwhich, int n, double* work, double* sig,
+                         int32_t* sweeps, hipStream_t s);
 int jacobi_max_sweeps();
 void launch_svd_scatter(const SvdScatter* ditems, int nitems, const SvdCol* dcols, const double* work, double* out,
                         hipStream_t s);

@@ -21,7 +21,7 @@
 namespace qsx {
 namespace {
 
-constexpr int SVD_NT = 1024;          // threads per workgroup of k_svd_finalize
+constexpr int SVD_NT = 1024;          // threads per workgroup of k_svd_finalize and k_jacobi_whole
 constexpr int SVD_NT_LDS = 512;       // threads per workgroup of k_jacobi_lds
 constexpr int SVD_NT_CROSS = 256;     // threads per workgroup of k_jacobi_cross
 constexpr int SVD_NT_BLOCK = 512;     // threads per workgroup of the block steps
@@ -215,18 +215,25 @@ __device__ __forceinline__ bool jacobi_pairs_m(double* A, double* V, int np, int
   return jacobi_pairs<NT, 0, CROSS>(A, V, np, nq, m, n, tol, flag);
 }
 
-constexpr int kColSplit = 16;  // one-wave workgroups a block's columns are dealt to (gather, scatter)
+// one-wave workgroups a block is dealt to (gather, scatter): whole columns, or
+// parts of columns where there are fewer columns (orthoQS of one 20223 x 1
+// matrix with its rows on one wave / on 16: 0.65 / 0.40 ms)
+constexpr int kColSplit = 16;
+__device__ __forceinline__ int col_parts(int ncols) { return max(1, (int)gridDim.y / max(1, ncols)); }
 
 // zero-padded group matrices: block e (d1 x d2, column-major) goes to
 // row i0, column j0 of its matrix (leading dim ld), transposed when trans
 __global__ __launch_bounds__(64) void k_svd_gather(const SvdGather* __restrict__ items, const double* __restrict__ src,
                                                     double* __restrict__ work) {
   const SvdGather it = items[blockIdx.x];
-  for (int j = blockIdx.y; j < it.d2; j += gridDim.y)
-    for (int i = threadIdx.x; i < it.d1; i += 64) {
+  const int parts = col_parts(it.d2);
+  for (int c = blockIdx.y; c < it.d2 * parts; c += gridDim.y) {
+    const int j = c / parts;
+    for (int i = 64 * (c % parts) + threadIdx.x; i < it.d1; i += 64 * parts) {
       const int64_t d = it.trans ? it.dst_off + j + (int64_t)i * it.ld : it.dst_off + i + (int64_t)j * it.ld;
       work[d] = src[it.src_off + (int64_t)j * it.d1 + i] * it.scale;
     }
+  }
 }
 
 // ---------------------------------------------------------------- n x n Jacobi
@@ -647,6 +654,46 @@ __global__ __launch_bounds__(SVD_NT_CROSS) void k_jacobi_cross(const SvdGroup* _
   if (threadIdx.x == 0) rot[sweep * ngroups + st.grp] = 1;
 }
 
+// all sweeps of an m x n matrix with m n + n^2 <= SVD_LDS_DOUBLES (checked by
+// the host) in one workgroup's LDS: a launch, where k_jacobi_block takes an
+// upload, n block steps and a wait per sweep, and at least four columns' room
+// (a single column of 10112 .. 20223 rows fits only here).  orthoQS of one
+// 2000 x 8 matrix, this kernel / column blocks: 0.76 / 1.12 ms.
+__global__ __launch_bounds__(SVD_NT) void k_jacobi_whole(const SvdItem* __restrict__ items,
+                                                         const int32_t* __restrict__ which,
+                                                         double* __restrict__ work, double* __restrict__ sig,
+                                                         int32_t* __restrict__ sweeps) {
+  __shared__ double lds[SVD_LDS_DOUBLES];
+  __shared__ int rotated;
+  const SvdItem it = items[which[blockIdx.x]];
+  const int m = it.m, n = it.n;  // m >= n >= 1
+  const int tid = threadIdx.x;
+  double* A = lds;
+  double* V = lds + m * n;
+  for (int e = tid; e < m * n; e += SVD_NT) A[e] = work[it.a_off + e];
+  for (int e = tid; e < n * n; e += SVD_NT) V[e] = e % (n + 1) == 0 ? 1.0 : 0.0;
+  __syncthreads();
+  int sw = 0;
+  for (; sw < SVD_MAX_SWEEPS; ++sw)
+    if (!jacobi_pairs<SVD_NT, 0, false>(A, V, n, 0, m, n, jacobi_tol(m, sw), &rotated)) break;
+  // sigma_j = |a_j|, u_j = a_j / sigma_j (a zero column stays zero)
+  const int seg = tid / SVD_SEG, lane = tid % SVD_SEG;
+  for (int j = seg; j < n; j += SVD_NT / SVD_SEG) {
+    double* aj = A + j * m;
+    double s2 = 0.0;
+    for (int i = lane; i < m; i += SVD_SEG) s2 += aj[i] * aj[i];
+    s2 = seg_sum(s2);
+    const double sg = sqrt(s2);
+    const double inv = sg > 0.0 ? 1.0 / sg : 0.0;
+    for (int i = lane; i < m; i += SVD_SEG) aj[i] *= inv;
+    if (lane == 0) sig[it.s_off + j] = sg;
+  }
+  __syncthreads();
+  for (int e = tid; e < m * n; e += SVD_NT) work[it.a_off + e] = A[e];
+  for (int e = tid; e < n * n; e += SVD_NT) work[it.v_off + e] = V[e];
+  if (tid == 0) sweeps[blockIdx.x] = sw;
+}
+
 // one step of the block one-sided Jacobi of a group matrix too large for
 // LDS: the columns of block P = [p0,p1) (and of block Q = [q0,q1)) and
 // their columns of V are staged in LDS; the pairs within P (q0 == q1) or
@@ -727,10 +774,12 @@ __global__ __launch_bounds__(64) void k_svd_scatter(const SvdScatter* __restrict
                                                     const SvdCol* __restrict__ cols, const double* __restrict__ work,
                                                     double* __restrict__ out) {
   const SvdScatter it = items[blockIdx.x];
-  for (int c = blockIdx.y; c < it.ncols; c += gridDim.y) {
+  const int parts = col_parts(it.ncols);
+  for (int k = blockIdx.y; k < it.ncols * parts; k += gridDim.y) {
+    const int c = k / parts;
     const SvdCol col = cols[it.col0 + c];
     const double* x = work + it.src_off + (int64_t)col.col * it.ld;
-    for (int r = threadIdx.x; r < it.rows; r += 64)
+    for (int r = 64 * (k % parts) + threadIdx.x; r < it.rows; r += 64 * parts)
       out[it.dst_off + r + (int64_t)c * it.rows] = x[r] * col.scale * it.scale;
   }
 }
@@ -755,6 +804,13 @@ void launch_jacobi_cross(const SvdGroup* dgroups, int ngroups, const SvdBlockSte
   if (nsteps <= 0) return;
   hipLaunchKernelGGL(k_jacobi_cross, dim3(nsteps), dim3(SVD_NT_CROSS), 0, s, dgroups, ngroups, dsteps, work, rot,
                      sweep);
+  QSX_HIP(hipGetLastError());
+}
+
+void launch_jacobi_whole(const SvdItem* ditems, const int32_t* dwhich, int n, double* work, double* sig,
+                         int32_t* sweeps, hipStream_t s) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_jacobi_whole, dim3(n), dim3(SVD_NT), 0, s, ditems, dwhich, work, sig, sweeps);
   QSX_HIP(hipGetLastError());
 }
 
