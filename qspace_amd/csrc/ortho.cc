@@ -151,6 +151,29 @@ struct OrthoResult {
 OrthoResult ortho_fused(const qsx_tensor* pt, const TensorDesc& P, int Nkmin, int64_t Nkeep, double stol,
                         const char* itag);
 
+// Group matrices up to SVD_QR_MAX_M x SVD_QR_MAX_N are reduced by QR before the
+// sweeps, unless all of a call are small: these are swept as they are, in one
+// workgroup's LDS each, since two QRs are a chain of 16 columns' reflectors at
+// least and four launches, as long as their sweeps.  orthoQS, ms, QR / as it is,
+// of one m x n matrix and of 12 in a call (values over six decades; random ones
+// in brackets):
+//   1000 x 4   0.36 / 0.30 (0.36 / 0.33)   0.53 / 0.40 (0.52 / 0.41)
+//   500 x 6    0.31 / 0.30 (0.32 / 0.32)   0.46 / 0.39 (0.47 / 0.41)
+//   1000 x 8   0.38 / 0.41 (0.39 / 0.50)   0.61 / 0.61 (0.61 / 0.69)
+//   500 x 10   0.34 / 0.39 (0.36 / 0.43)   0.53 / 0.48 (0.53 / 0.57)
+//   500 x 12   0.34 / 0.42 (0.37 / 0.52)   0.54 / 0.53 (0.54 / 0.63)
+//   250 x 20   0.40 / 0.40 (0.45 / 0.50)   0.59 / 0.51 (0.63 / 0.62)
+//   64 x 24    0.37 / 0.35 (0.41 / 0.41)   0.45 / 0.44 (0.49 / 0.49)
+//   250 x 24   0.41 / 0.44 (0.45 / 0.58)   0.61 / 0.57 (0.65 / 0.69)
+//   32 x 32    0.38 / 0.40 (0.42 / 0.49)
+// Beside larger matrices, which take the QRs, they do better in their shadow:
+// the SU(2) MPS tensor of 17 groups up to 128 x 64 takes 1.28 ms with all of them
+// reduced, 1.45 ms without the small ones.
+bool small_matrix(int64_t m, int64_t n) { return n <= 6 || (n <= 24 && m * n <= 5120); }
+bool use_qr(int64_t m, int64_t n, bool all_small) {
+  return m <= SVD_QR_MAX_M && n <= SVD_QR_MAX_N && !(all_small && small_matrix(m, n));
+}
+
 OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep, double stol, const char* itag) {
   if (pt && pt->data_im) fail(QSX_ERR_UNSUPPORTED, "orthoQS: complex data not supported (real QSpaces only)");
   TensorDesc P = make_desc(pt, "PSI");
@@ -257,6 +280,7 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
     work += (n + 15) & ~(int64_t)15;
     return o;
   };
+  const bool all_small = std::all_of(G.begin(), G.end(), [](const Group& b) { return small_matrix(b.m, b.n); });
   for (auto& b : G) {
     if (b.n == 0) continue;
     if (b.n > INT32_MAX || b.m > INT32_MAX) fail(QSX_ERR_UNSUPPORTED, "orthoQS: group matrix too large");
@@ -271,7 +295,7 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
     it.s_off = b.s_off;
     it.m = (int32_t)b.m;
     it.n = (int32_t)b.n;
-    if (b.m <= SVD_QR_MAX_M && b.n <= SVD_QR_MAX_N) {
+    if (use_qr(b.m, b.n, all_small)) {
       SvdGroup q{};
       q.a = b.a_off;
       q.v = b.v_off;
@@ -431,38 +455,46 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
     nbk.push_back((int32_t)nb);
     cbk.push_back((int32_t)cb);
   }
-  std::vector<UploadPart> up;
-  auto put = [&](auto& v) {
-    using T = typename std::decay_t<decltype(v)>::value_type;
-    T* d = (T*)fr.add(sizeof(T) * std::max<size_t>(1, v.size()));
-    if (!v.empty()) up.push_back({d, v.data(), sizeof(T) * v.size()});
-    return d;
+  // the descriptor lists in one device buffer, filled by one copy, and the
+  // kernels' small arrays behind them: with a buffer and a copy for each, their
+  // allocation took longer than the sweeps of small groups
+  std::vector<char> desc;
+  auto put = [&](const auto& v) {  // byte offset of the list
+    const size_t o = (desc.size() + 255) / 256 * 256;
+    desc.resize(o + sizeof(v[0]) * v.size());
+    if (!v.empty()) std::memcpy(desc.data() + o, v.data(), sizeof(v[0]) * v.size());
+    return o;
   };
-  SvdItem* ditems = put(items);
-  SvdGather* dgath = put(gath);
-  int32_t* dwhole = put(whole);
-  int32_t* dbig = put(big);
-  SvdGroup* dqr = put(qr);
-  SvdQr* dqr1 = put(qr1);
-  SvdQr* dqr2 = put(qr2);
-  SvdApply* dapp = put(app);
-  SvdItem* dunit = put(unit);
-  int32_t* dunitidx = put(unitidx);
-  int32_t* dsmall = put(small);
-  SvdBlockStep* drsteps = put(rsteps);
-  int32_t* dperm = (int32_t*)fr.add(sizeof(int32_t) * std::max<int64_t>(1, nperm));
-  int32_t* dexpo = (int32_t*)fr.add(sizeof(int32_t) * std::max<size_t>(1, qr.size()));
-  int32_t* dsw = (int32_t*)fr.add(sizeof(int32_t) * std::max<size_t>(1, small.size() + whole.size()));
+  const size_t o_items = put(items), o_gath = put(gath), o_whole = put(whole), o_big = put(big), o_qr = put(qr),
+               o_qr1 = put(qr1), o_qr2 = put(qr2), o_app = put(app), o_unit = put(unit), o_unitidx = put(unitidx),
+               o_small = put(small), o_rsteps = put(rsteps);
+  size_t nbytes = desc.size();
+  auto after = [&](size_t n) {  // n int32 beyond the lists
+    const size_t o = (nbytes + 255) / 256 * 256;
+    nbytes = o + sizeof(int32_t) * n;
+    return o;
+  };
   const size_t nrot = (size_t)jacobi_max_sweeps() * qr.size();
-  int32_t* drot = (int32_t*)fr.add(sizeof(int32_t) * std::max(nrot, items.size()));
+  const size_t o_perm = after(nperm), o_expo = after(qr.size()), o_sw = after(small.size() + whole.size()),
+               o_rot = after(std::max(nrot, items.size()));
+  char* dd = (char*)fr.add(nbytes);
+  SvdItem* ditems = (SvdItem*)(dd + o_items);
+  SvdGather* dgath = (SvdGather*)(dd + o_gath);
+  int32_t *dwhole = (int32_t*)(dd + o_whole), *dbig = (int32_t*)(dd + o_big);
+  SvdGroup* dqr = (SvdGroup*)(dd + o_qr);
+  SvdQr *dqr1 = (SvdQr*)(dd + o_qr1), *dqr2 = (SvdQr*)(dd + o_qr2);
+  SvdApply* dapp = (SvdApply*)(dd + o_app);
+  SvdItem* dunit = (SvdItem*)(dd + o_unit);
+  int32_t *dunitidx = (int32_t*)(dd + o_unitidx), *dsmall = (int32_t*)(dd + o_small);
+  SvdBlockStep* drsteps = (SvdBlockStep*)(dd + o_rsteps);
+  int32_t *dperm = (int32_t*)(dd + o_perm), *dexpo = (int32_t*)(dd + o_expo), *dsw = (int32_t*)(dd + o_sw),
+          *drot = (int32_t*)(dd + o_rot);
   upload_packed(P, P.hdata, dpsi.p, s);
-  upload_many(up, s);
+  upload_many({{dd, desc.data(), desc.size()}}, s);
   Timer tm(s);
   launch_fill_zero(dwork.p, work, s);
   launch_svd_gather(dgath, (int)gath.size(), dpsi.p, dwork.p, s);
-  launch_svd_qr(dqr1, (int)qr1.size(), maxrows, dwork.p, dperm, dexpo, s);
-  launch_svd_qr(dqr2, (int)qr2.size(), SVD_QR_MAX_N, dwork.p, dperm, dexpo, s);
-  // the groups in LDS run on the side stream, beside the block steps
+  // the groups in LDS run on the side stream, beside the QRs and the block steps
   hipStream_t s2 = side_stream();
   struct Ev {
     hipEvent_t e = nullptr;
@@ -478,10 +510,20 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
       (void)hipStreamSynchronize(b);
     }
   } drain{s, s2};
-  QSX_HIP(hipEventRecord(ready.e, s));
-  QSX_HIP(hipStreamWaitEvent(s2, ready.e, 0));
-  launch_jacobi_lds(dqr, dsmall, (int)small.size(), dwork.p, dsw, s2);
-  launch_jacobi_whole(ditems, dwhole, (int)whole.size(), dwork.p, dsig.p, dsw + small.size(), s2);
+  auto fork = [&]() {  // s2 follows what s holds so far
+    QSX_HIP(hipEventRecord(ready.e, s));
+    QSX_HIP(hipStreamWaitEvent(s2, ready.e, 0));
+  };
+  if (!whole.empty()) {
+    fork();
+    launch_jacobi_whole(ditems, dwhole, (int)whole.size(), dwork.p, dsig.p, dsw + small.size(), s2);
+  }
+  launch_svd_qr(dqr1, (int)qr1.size(), maxrows, dwork.p, dperm, dexpo, s);
+  launch_svd_qr(dqr2, (int)qr2.size(), SVD_QR_MAX_N, dwork.p, dperm, dexpo, s);
+  if (!small.empty()) {
+    fork();
+    launch_jacobi_lds(dqr, dsmall, (int)small.size(), dwork.p, dsw, s2);
+  }
   QSX_HIP(hipEventRecord(done.e, s2));
   int maxsw = 0;
   if (!big.empty()) {

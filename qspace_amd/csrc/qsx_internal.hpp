@@ -398,10 +398,10 @@ void launch_fill_zero(double* p, int64_t n, hipStream_t s);
 // (svd.hip, svdqr.hip) group matrices of the truncation, one-sided Jacobi SVD,
 // result blocks.  A group matrix is stored m x n column-major with m >= n
 // (the transpose of a wide matrix).  Up to SVD_QR_MAX_M x SVD_QR_MAX_N it is
-// reduced to an n x n triangle by QR first and decomposed there, in one
-// workgroup's LDS for n <= SVD_LDS_N and by rounds of column blocks beyond;
-// another one is decomposed as it is, in one workgroup's LDS when m n + n^2 <=
-// SVD_LDS_DOUBLES, by column-block steps beyond.
+// reduced to an n x n triangle by QR first (unless all are small: use_qr in
+// ortho.cc) and decomposed there, in one workgroup's LDS for n <= SVD_LDS_N and
+// by rounds of column blocks beyond; another one is decomposed as it is, in one
+// workgroup's LDS when m n + n^2 <= SVD_LDS_DOUBLES, by column-block steps beyond.
 constexpr int SVD_QR_MAX_M = 1024;
 constexpr int SVD_QR_MAX_N = 256;
 constexpr int SVD_LDS_N = 96;         // 2 n (n + 8) doubles fit a workgroup's LDS

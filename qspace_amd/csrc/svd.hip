@@ -9,10 +9,11 @@
 // pairs; a sweep visits every pair once, in steps of disjoint pairs that run
 // in parallel.  At the end x_j = sigma_j u_j and the accumulated rotations
 // are W.  Matrices of up to SVD_QR_MAX_M x SVD_QR_MAX_N are reduced to an
-// n x n triangle first (svdqr.hip); k_jacobi_lds runs all sweeps of one with
-// n <= SVD_LDS_N in a workgroup's LDS, k_jacobi_cross one round of column
-// blocks of a larger one.  Still larger matrices take k_jacobi_block, on the
-// m x n matrix itself.
+// n x n triangle first (svdqr.hip) unless small; k_jacobi_lds runs all sweeps of
+// one with n <= SVD_LDS_N in a workgroup's LDS, k_jacobi_cross one round of
+// column blocks of a larger one.  Other matrices are swept as they are: in a
+// workgroup's LDS where they fit (k_jacobi_whole: small ones, and few columns
+// of more than SVD_QR_MAX_M rows), by k_jacobi_block where they do not.
 #include <cfloat>
 
 #include "qsx_internal.hpp"
@@ -206,12 +207,19 @@ __device__ __forceinline__ bool jacobi_pairs(double* A, double* V, int np, int n
   return any;
 }
 
-// the variant for column length m (longer than SVD_QR_MAX_N, or of more rows
-// than SVD_QR_MAX_M)
+// the variant for column length m; CROSS: m is longer than SVD_QR_MAX_N
 template <int NT, bool CROSS>
 __device__ __forceinline__ bool jacobi_pairs_m(double* A, double* V, int np, int nq, int m, int n, double tol,
                                                int* flag) {
-  if (m <= 512) return jacobi_pairs<NT, 32, CROSS>(A, V, np, nq, m, n, tol, flag);
+  if constexpr (!CROSS) {
+    if (m <= 16) return jacobi_pairs<NT, 1, CROSS>(A, V, np, nq, m, n, tol, flag);
+    if (m <= 32) return jacobi_pairs<NT, 2, CROSS>(A, V, np, nq, m, n, tol, flag);
+    if (m <= 64) return jacobi_pairs<NT, 4, CROSS>(A, V, np, nq, m, n, tol, flag);
+    if (m <= 128) return jacobi_pairs<NT, 8, CROSS>(A, V, np, nq, m, n, tol, flag);
+    if (m <= 256) return jacobi_pairs<NT, 16, CROSS>(A, V, np, nq, m, n, tol, flag);
+  }
+  if constexpr (NT <= 512)  // registers for 32 elements per lane
+    if (m <= 512) return jacobi_pairs<NT, 32, CROSS>(A, V, np, nq, m, n, tol, flag);
   return jacobi_pairs<NT, 0, CROSS>(A, V, np, nq, m, n, tol, flag);
 }
 
@@ -675,7 +683,7 @@ __global__ __launch_bounds__(SVD_NT) void k_jacobi_whole(const SvdItem* __restri
   __syncthreads();
   int sw = 0;
   for (; sw < SVD_MAX_SWEEPS; ++sw)
-    if (!jacobi_pairs<SVD_NT, 0, false>(A, V, n, 0, m, n, jacobi_tol(m, sw), &rotated)) break;
+    if (!jacobi_pairs_m<SVD_NT, false>(A, V, n, 0, m, n, jacobi_tol(m, sw), &rotated)) break;
   // sigma_j = |a_j|, u_j = a_j / sigma_j (a zero column stays zero)
   const int seg = tid / SVD_SEG, lane = tid % SVD_SEG;
   for (int j = seg; j < n; j += SVD_NT / SVD_SEG) {

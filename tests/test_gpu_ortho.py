@@ -167,10 +167,11 @@ def test_ortho_rank_deficient_groups(gpu):
 # the line beyond which the matrix itself is swept (n = 257, m = 1025) and, of
 # those, the ones in one workgroup's LDS (m n + n^2 <= 20224, among them the
 # single columns that no pair of column blocks has room for) and the first
-# beyond it
+# beyond it; small ones are swept as they are too (n <= 6, or n <= 24 and
+# m n <= 5120)
 SHAPES = [(1, 1), (2, 2), (5, 2), (16, 16), (17, 16), (40, 17), (33, 32), (96, 96), (97, 97), (130, 96), (128, 97),
           (129, 128), (140, 129), (256, 193), (257, 225), (256, 256), (513, 60), (600, 100), (1024, 33), (1025, 20),
-          (258, 257), (300, 1), (2000, 8), (2520, 8), (2521, 8), (1045, 19), (1046, 19), (10111, 1), (12000, 1), (20223, 1)]
+          (258, 257), (300, 1), (24, 24), (25, 25), (1024, 6), (1024, 7), (640, 8), (641, 8), (213, 24), (214, 24), (2000, 8), (2520, 8), (2521, 8), (1045, 19), (1046, 19), (10111, 1), (12000, 1), (20223, 1)]
 
 
 @pytest.mark.parametrize("kind", ["random", "graded", "deficient", "scaled"])
