@@ -273,6 +273,8 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   std::vector<SvdGather> gath;
   std::vector<SvdItem> items;
   std::vector<SvdGroup> qr;         // the groups reduced by QR
+  std::vector<int32_t> qritem;      // their items
+  std::vector<int> groff(1, 0);     // an item's range of gath
   std::vector<int32_t> whole, big;  // the others: in one workgroup's LDS, beyond it
   int64_t work = 0, nsig = 0, nperm = 0;
   auto take = [&](int64_t n) {  // buffers start at multiples of 16 doubles
@@ -311,6 +313,7 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
       q.c1 = take((int64_t)q.ldf * q.n16);
       q.c2 = take((int64_t)q.n16 * q.n16);
       qr.push_back(q);
+      qritem.push_back((int32_t)items.size());
     } else {
       (b.m * b.n + b.n * b.n <= SVD_LDS_DOUBLES ? whole : big).push_back((int32_t)items.size());
     }
@@ -342,6 +345,7 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
       if ((int64_t)gg.d1 * gg.d2 != P.numel(i)) fail(QSX_ERR_STRUCT, "orthoQS: block %d dims", i + 1);
       gath.push_back(gg);
     }
+    groff.push_back((int)gath.size());
   }
   if (nsig == 0) fail(QSX_ERR_ARG, "orthoQS: got empty SVD data");
   // the QR factorisations (all groups', then the second ones), the groups
@@ -442,18 +446,19 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   // groups beyond the QR's range and the LDS: block one-sided Jacobi over column blocks
   // of at most cb columns, two blocks (and their columns of V) staged in LDS
   // per workgroup
-  std::vector<int32_t> nbk, cbk;
-  for (int32_t i : big) {
+  auto col_blocks = [&](int32_t i, int& nb, int& cb) {
     const int64_t m = items[i].m, n = items[i].n;
     const int64_t cmax = SVD_LDS_DOUBLES / (2 * (m + n));
     if (cmax < 1) fail(QSX_ERR_UNSUPPORTED, "orthoQS: group matrix %lld x %lld too large", (long long)m, (long long)n);
-    int64_t nb = (n + cmax - 1) / cmax;
+    nb = (int)((n + cmax - 1) / cmax);
     nb += nb & 1;
     if (nb < 2) nb = 2;
-    const int64_t cb = (n + nb - 1) / nb;
+    cb = (int)((n + nb - 1) / nb);
     if (2 * cb * (m + n) > SVD_LDS_DOUBLES) fail(QSX_ERR_STRUCT, "orthoQS: internal column block too large");
-    nbk.push_back((int32_t)nb);
-    cbk.push_back((int32_t)cb);
+  };
+  for (int32_t i : big) {
+    int nb, cb;
+    col_blocks(i, nb, cb);
   }
   // the descriptor lists in one device buffer, filled by one copy, and the
   // kernels' small arrays behind them: with a buffer and a copy for each, their
@@ -526,7 +531,10 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   }
   QSX_HIP(hipEventRecord(done.e, s2));
   int maxsw = 0;
-  if (!big.empty()) {
+  auto sweep_blocks = [&](const std::vector<int32_t>& big, const int32_t* dbig) {
+    if (big.empty()) return;
+    std::vector<int> nbk(big.size()), cbk(big.size());
+    for (size_t a = 0; a < big.size(); ++a) col_blocks(big[a], nbk[a], cbk[a]);
     launch_svd_init_v(ditems, dbig, (int)big.size(), dwork.p, s);
     std::vector<int> active(big.size());
     std::iota(active.begin(), active.end(), 0);
@@ -590,9 +598,10 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
       active.swap(next);
     }
     if (!active.empty()) fail(QSX_ERR_ARG, "orthoQS: block Jacobi SVD did not converge in %d sweeps", sw);
-    maxsw = sw;
+    maxsw = std::max(maxsw, sw);
     launch_svd_finalize(ditems, dbig, (int)big.size(), dwork.p, dsig.p, s);
-  }
+  };
+  sweep_blocks(big, dbig);
   if (!mid.empty()) {
     launch_svd_init_v(dunit, dunitidx, (int)unit.size(), dwork.p, s);
     QSX_HIP(hipMemsetAsync(drot, 0, sizeof(int32_t) * nrot, s));
@@ -622,13 +631,38 @@ OrthoResult ortho_oneshot(const qsx_tensor* pt, int K, int Nkmin, int64_t Nkeep,
   launch_svd_applyq(dapp, (int)app.size(), maxrows, dwork.p, dperm, s);
   std::vector<double> sig(nsig);
   std::vector<int32_t> sweeps(small.size() + whole.size());
-  QSX_HIP(hipMemcpyAsync(sig.data(), dsig.p, sizeof(double) * nsig, hipMemcpyDeviceToHost, s));
-  if (!sweeps.empty())
-    QSX_HIP(hipMemcpyAsync(sweeps.data(), dsw, sizeof(int32_t) * sweeps.size(), hipMemcpyDeviceToHost, s));
-  QSX_HIP(hipStreamSynchronize(s));
-  for (int x : sweeps) {
-    if (x >= jacobi_max_sweeps()) fail(QSX_ERR_ARG, "orthoQS: Jacobi SVD did not converge in %d sweeps", x);
-    maxsw = std::max(maxsw, x + 1);
+  auto download = [&](const int32_t* dsweeps) {
+    QSX_HIP(hipMemcpyAsync(sig.data(), dsig.p, sizeof(double) * nsig, hipMemcpyDeviceToHost, s));
+    if (!sweeps.empty())
+      QSX_HIP(hipMemcpyAsync(sweeps.data(), dsweeps, sizeof(int32_t) * sweeps.size(), hipMemcpyDeviceToHost, s));
+    QSX_HIP(hipStreamSynchronize(s));
+    for (int x : sweeps) {
+      if (x >= jacobi_max_sweeps()) fail(QSX_ERR_ARG, "orthoQS: Jacobi SVD did not converge in %d sweeps", x);
+      maxsw = std::max(maxsw, x + 1);
+    }
+  };
+  download(dsw);
+  // A NaN or an infinity goes through the reflectors into every column, where
+  // rotations leave the columns without one alone: a group that came out so is
+  // assembled again and swept as it is
+  std::vector<int32_t> redo, redo_big;
+  for (size_t i = 0; i < qr.size(); ++i) {
+    const double* x = sig.data() + qr[i].s;
+    if (std::all_of(x, x + qr[i].n, [](double v) { return std::isfinite(v); })) continue;
+    const int64_t mn = (int64_t)qr[i].m * qr[i].n, nn = (int64_t)qr[i].n * qr[i].n;
+    const int32_t k = qritem[i];
+    (mn + nn <= SVD_LDS_DOUBLES ? redo : redo_big).push_back(k);
+    launch_fill_zero(dwork.p + items[k].a_off, mn, s);
+    launch_svd_gather(dgath + groff[k], groff[k + 1] - groff[k], dpsi.p, dwork.p, s);
+  }
+  if (!redo.empty() || !redo_big.empty()) {
+    const size_t n = redo.size(), nb = redo_big.size();
+    int32_t* dredo = (int32_t*)fr.add(sizeof(int32_t) * (2 * n + nb));  // indices, then sweeps
+    upload_many({{dredo, redo.data(), sizeof(int32_t) * n}, {dredo + n, redo_big.data(), sizeof(int32_t) * nb}}, s);
+    launch_jacobi_whole(ditems, dredo, (int)n, dwork.p, dsig.p, dredo + n + nb, s);
+    sweep_blocks(redo_big, dredo + n);
+    sweeps.assign(n, 0);
+    download(dredo + n + nb);
   }
 
   // ---- truncation (dmrgTruncate)

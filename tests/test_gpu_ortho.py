@@ -214,3 +214,28 @@ def test_svd_shapes(gpu, kind, wide):
         assert np.linalg.norm(U @ V.T - M) <= tol * np.linalg.norm(M)
         if kind != "deficient":  # columns of zero singular values are zero
             assert np.abs(U.T @ U - np.eye(n)).max() <= tol
+
+
+# group matrices that are swept as they are (8 x 6), in LDS after the QRs (60 x
+# 40), by rounds of column blocks (130 x 110) and, beyond the QRs, as they are
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("m,n", [(8, 6), (60, 40), (130, 110), (300, 200), (300, 260)])
+def test_svd_non_finite(gpu, m, n, bad):
+    """a NaN or an infinity in one column of a group leaves the other columns'
+    decomposition and the other groups finite.  Tolerance as in
+    test_svd_shapes."""
+    rng = np.random.default_rng(m + n)
+    M, other = rng.standard_normal((m, n)), rng.standard_normal((50, 40))
+    M[m // 3, n // 2] = bad
+    P = Q.QSpace([np.array([[0], [1]]), np.array([[0], [1]])], [M, other], "A", ["L", "R*"])
+    A1, A2, info = Q.orthoQS(P, 1, stol=0.0)
+    svd = np.asarray(info["svd"])
+    fin = np.sort(svd[np.isfinite(svd)])
+    ref = np.sort(np.concatenate([np.linalg.svd(np.delete(M, n // 2, 1), compute_uv=False),
+                                  np.linalg.svd(other, compute_uv=False)]))
+    tol = 8.0 * np.sqrt(60.0 * (m + n)) * np.finfo(float).eps
+    assert len(svd) == n + 40 and len(fin) == n + 39
+    assert np.abs(fin - ref).max() <= tol * ref[-1]
+    U = A1.data[0][:, np.isfinite(A1.data[0]).all(axis=0)]
+    assert U.shape == (m, n - 1) and np.abs(U.T @ U - np.eye(n - 1)).max() <= tol
+    assert np.linalg.norm(A1.data[1] @ A2.data[1].T - other) <= tol * np.linalg.norm(other)
