@@ -212,23 +212,23 @@ __global__ __launch_bounds__(RT) void k_gs_update_mdot(double* __restrict__ w, c
 // / beta with beta^2 = |w|^2 - sum_j c[j]^2, the squared norm of the update
 // for orthonormal V_j.  After a first pass the c[j] are at rounding level
 // relative to |w| and the difference is exact to rounding; when they are
-// not (|c|^2 > lim |w|^2) dst = 0 and beta = brk: 0 with lim = 1/2 after a
-// second pass (w is rounding noise inside span V, a breakdown), -1 with a
-// smaller lim where this is the only full pass (w had components in span V
+// not (|c|^2 > lim |w|^2) dst = 0 and beta = 0 with lim = 1/2 after a
+// second pass (w is rounding noise inside span V, a breakdown), beta = -|w| with
+// a smaller lim where this is the only full pass (w had components in span V
 // after all, and one pass leaves more than rounding of them).  Every block sums
 // the partials and the squares in the same order.
 __global__ __launch_bounds__(RT) void k_gs_update_normalize(const double* __restrict__ w,
                                                              const double* __restrict__ V, int64_t ldv,
                                                              const double* __restrict__ pin, int m, int64_t n,
                                                              double* __restrict__ dst, double* __restrict__ beta,
-                                                             double lim, double brk) {
+                                                             double lim, bool only) {
   __shared__ double c[kMaxM + 1];
   __shared__ double inv;
   sum_coefficients(pin, m + 1, c);
   if (threadIdx.x == 0) {
     double cs = 0;
     for (int j = 0; j < m; ++j) cs += c[j] * c[j];
-    const double b = cs <= lim * c[m] ? sqrt(c[m] - cs) : brk;
+    const double b = cs <= lim * c[m] ? sqrt(c[m] - cs) : only ? -sqrt(c[m]) : 0.0;
     inv = b > 0 ? 1.0 / b : 0.0;
     if (blockIdx.x == 0 && beta) *beta = b;
   }
@@ -411,7 +411,7 @@ void vec_gs_update_normalize(const double* w, const double* V, int64_t ldv, cons
   if (m <= 0) return;
   if (m > kMaxM) fail_vec(m);
   hipLaunchKernelGGL(k_gs_update_normalize, dim3(grid_for(n)), dim3(RT), 0, s, w, V, ldv, pin, m, n, dst, beta,
-                     only ? kOnePassLim : 0.5, only ? -1.0 : 0.0);
+                     only ? kOnePassLim : 0.5, only);
 }
 
 void vec_scale_norm_partial(const double* src, const double* w, double* dst, int64_t n, double* partial,

@@ -30,7 +30,7 @@ void vec_gs_local_mdot(double* w, const double* V, int64_t ldv, const double* pi
 // dst = (w - V c(pin)) / beta, beta^2 = |w|^2 - |c|^2 from the partials pin
 // (m coefficient sets, then |w|^2), written to *beta if given.  The second of
 // two passes: beta = 0 and dst = 0 when |c|^2 > |w|^2 / 2 (w is rounding noise
-// inside span V).  The only full pass: beta = -1 and dst = 0 when |c|^2 >
+// inside span V).  The only full pass: beta = -|w| and dst = 0 when |c|^2 >
 // kOnePassLim |w|^2 (up to there the result's components in span V are
 // rounding of |w|, as after a second pass; the caller makes two passes)
 constexpr double kOnePassLim = 0.01;

@@ -312,6 +312,28 @@ def test_eigensolvers_vs_numpy_krylov(gpu, hconj, niter):
     assert np.abs(H.davidson(x0, niter)[1] - ritz).max() < tol
 
 
+@pytest.mark.parametrize("kw,niters", [(dict(Dstar=8, mu=0.6, sigma=0.3, dmax=3), (14, 15, 16, 40)),
+                                       (dict(Dstar=150, mu=1.5, sigma=0.5, dmax=12), (20, 70))])
+@pytest.mark.parametrize("hconj", [1, 0])
+def test_eigensolver_passes(gpu, capfd, kw, niters, hconj):
+    """which steps the eigensolvers make with two Gram-Schmidt passes, as they
+    report it: none for a symmetric operator, also where the Krylov space ends
+    (N = 15) within the steps asked for, which only ends T there; from some step
+    on for one that is not symmetric.  Either way V stays orthonormal, so the
+    Ritz vector V y has norm 1 to rounding (70 vectors: 1e-14)."""
+    H = Q.HPsi(*gen.heis_hpsi(seed=25, **kw), hconj=hconj, verbose=2)
+    x0 = np.random.RandomState(2).standard_normal(H.N)
+    for niter in niters:
+        for solver in (H.lanczos, H.davidson):
+            capfd.readouterr()
+            gs = solver(x0, niter)[2]
+            err = capfd.readouterr().err
+            ends = solver == H.lanczos and hconj and H.N <= niter
+            assert ("the Krylov space ends after %d vectors" % H.N in err) == ends, err
+            assert ("two passes from step" in err) == (not hconj), err
+            assert abs(np.sqrt((H.weights() * gs) @ gs) - 1.0) < 1e-14, (solver.__name__, niter)
+
+
 def test_lanczos_invariant_start(gpu):
     """Lanczos started on an exact eigenvector (the highest, positive
     eigenvalue of a small Heisenberg operator): the Krylov space is
