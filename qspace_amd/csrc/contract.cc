@@ -739,14 +739,22 @@ static std::vector<WorkTarget> plan_targets(const CtrPlan& P) {
 // SU(2)) in 1x1-fragment tiles shared beyond 8 MFMAs / 2x2 beyond 8 / 2x2 beyond
 // 64: 345 MFMAs a plan 8.1 / 9.3 / 12.0, 3.2e3 8.8 / 11.6 / 16.3, 5.0e3 9.5 / 11.7
 // / 16.4, 1.0e4 13.1 / 12.9 / 16.8, 1.4e4 14.5 / 13.1 / 17.2.  (Between 24 and 44
-// a SIMD as in stage 1 of H*psi.)  A plan used once also pays for building its
-// list, about 0.08 us an item: up to 4x4 fragments a tile; environment update of
-// a U(1) MPS (F = 1.0e4, 5.0e4, 5.7e3; whole call) 3.9 ms against 7.3 ms with 2x2
-// tiles, of which the kernels are 0.12 and 0.08 ms.  Sharing changes the order of
+// a SIMD as in stage 1 of H*psi.)  A plan used a few times only (runs > 0) also
+// pays for building its list, 0.03 us an item: up to 4x4 fragments a tile where
+// that saves more than it adds to the executions.  No wave shares such a tile;
+// the longest takes 0.043 us an MFMA alone, and smaller tiles take that for an
+// average SIMD's MFMAs at least.  List, its upload and the kernel, ms, 2x2 / 4x4
+// tiles: one block of 1100 x 1100, k = 300 0.22 / 0.11, 1000 0.27 / 0.23, 2000 0.38 /
+// 0.39, 4000 0.57 / 0.71, 10000 1.15 / 1.67; complex (four executions) k = 200 0.35 /
+// 0.26, 500 0.45 / 0.47, 1000 0.62 / 0.80; 2048^3 1.10 / 0.48; 20 blocks of 300 x 300,
+// k = 1200 0.52 / 0.28; 150 of 100 x 100, k = 200 0.37 / 0.14.
+// Environment update of a U(1) MPS (F = 1.0e4, 5.0e4, 5.7e3; whole call) 3.9 ms
+// against 7.3 ms with 2x2 tiles.  Sharing changes the order of
 // a tile's sum: against 80-bit sums the environment step's mean relative errors
 // are 1.6e-16 and 2.6e-16 (L.A, X.conj(A)), unshared 2.1e-16 and 3.3e-16 -- whose
 // sequential order FP64 numpy has as well, so that it differs from that less.
-static void default_policy(CtrPlan& P, bool once) {
+constexpr double kItemUs = 0.03, kMfmaUs = 0.043;
+static void default_policy(CtrPlan& P, int runs) {
   double mfma = 0, frags = 0;
   for (int t = 0; t < P.nT; ++t) {
     const double f = (double)((P.M[t] + 15) / 16) * ((P.N[t] + 15) / 16);
@@ -758,7 +766,21 @@ static void default_policy(CtrPlan& P, bool once) {
   const double mean = mfma / 1024;
   P.policy.wave_max = mean < 8 ? 1 : 2;
   P.policy.group_mfma = mean < 24 ? 8 : mean < 44 ? 32 : 64;
-  if (once && frags > 4096) P.policy.wave_max = 4;
+  if (!runs || frags <= 4096) return;
+  const int mx = P.policy.wave_max;
+  double items = 0, items4 = 0, longest = 0;
+  for (int t = 0; t < P.nT; ++t) {
+    const int mf = (P.M[t] + 15) / 16, nf = (P.N[t] + 15) / 16;
+    if (!mf || !nf) continue;
+    double steps = 0;
+    for (int64_t p = P.pseg[t]; p < P.pseg[t + 1]; ++p) steps += (P.pairs[p].K + 3) / 4;
+    const double tiles = (double)((mf + mx - 1) / mx) * ((nf + mx - 1) / mx);
+    const double mfma = steps * mf * nf / tiles;  // of a tile; a shared one is an item per wave
+    items += mfma > P.policy.group_mfma && steps >= 4 ? 4 * tiles : tiles;
+    items4 += (double)((mf + 3) / 4) * ((nf + 3) / 4);
+    longest = std::max(longest, steps * std::min(mf, 4) * std::min(nf, 4));
+  }
+  if (kItemUs * (items - items4) > runs * kMfmaUs * std::max(0.0, longest - mean)) P.policy.wave_max = 4;
 }
 
 void plan_upload(CtrPlan& P) {
@@ -767,6 +789,9 @@ void plan_upload(CtrPlan& P) {
   const std::vector<WorkTarget> targets = plan_targets(P);
   P.work = build_work(targets, P.pairs, P.policy);
   clk.lap("build_work");
+  if (P.verbose >= 2)
+    fprintf(stderr, "qsx contract plan: %zu items, tiles of up to %d x %d fragments\n", P.work.items.size(),
+            P.policy.wave_max, P.policy.wave_max);
   for (void** q : {(void**)&P.dpairs, (void**)&P.ditems, (void**)&P.dreds, (void**)&P.dqueues, (void**)&P.dscratch}) {
     dev_free(*q);
     *q = nullptr;
@@ -846,7 +871,7 @@ std::unique_ptr<CtrPlan> plan_create(const qsx_tensor* A, const int32_t* ia, int
     fail(QSX_ERR_UNSUPPORTED, "split precision is available for H*psi plans only (QSX_MODE_SPLIT_BF16)");
   build_structure(*P, perm, nperm, o ? o->fermA : nullptr, o ? o->fermB : nullptr);
   PhaseClock clk{P->verbose, "contract plan"};
-  default_policy(*P, force & kPlanOnce);
+  default_policy(*P, force / kPlanOnce);
   if (upload) plan_upload(*P);
   clk.lap("work list + upload");
   return P;
@@ -1053,7 +1078,8 @@ static qsx_tensor_out* contract_oneshot_complex(const qsx_tensor* A, const int32
                                                 const qsx_tensor* B, const int32_t* ib, int nb, int conjB,
                                                 const int32_t* perm, int nperm, const qsx_opts* o) {
   hipStream_t s = default_stream();
-  auto P = plan_create(A, ia, na, conjA, B, ib, nb, conjB, perm, nperm, o, true, kPlanOnce);
+  auto P = plan_create(A, ia, na, conjA, B, ib, nb, conjB, perm, nperm, o, true,
+                       kPlanOnce * (A->data_im ? 2 : 1) * (B->data_im ? 2 : 1));
   const bool ai = P->A.hdata_im != nullptr, bi = P->B.hdata_im != nullptr;
   // the plan may have applied the missing-conj rule (contract_getIdxSet)
   const double sA = P->conjA ? -1.0 : 1.0, sB = P->conjB ? -1.0 : 1.0;

@@ -73,7 +73,7 @@ struct CtrPlan {
 // force: bit 0 / bit 1 -- give A / B a permuted copy in the orientation the
 // GEMM loads best (A as M x K, B as N x K: 16 consecutive rows / columns per
 // k) even when the native layout would do (plans of constant operands);
-// kPlanOnce: the plan is executed once
+// kPlanOnce * n: the plan is executed n times in all (without: many times)
 constexpr int kPlanOnce = 4;
 std::unique_ptr<CtrPlan> plan_create(const qsx_tensor* A, const int32_t* ia, int na, int conjA, const qsx_tensor* B,
                                      const int32_t* ib, int nb, int conjB, const int32_t* perm, int nperm,

@@ -611,3 +611,27 @@ def test_split_f32x3_vs_oracle(gpu, heis4000):
     assert abs(e_f32 - e_ref) < 1e-10 * abs(e_ref), (e_f32, e_ref)
     with pytest.raises(Q.QsxError):
         Q.HPsi(HL, psi, HR, hconj=1, mode="split_f32", nslices=4)
+
+
+@pytest.mark.parametrize("m,k,ngrp,cplx,tiles", [(1000, 64, 1, 0, 2), (1100, 64, 1, 0, 4), (1100, 1000, 1, 0, 4),
+                                                 (1100, 3000, 1, 0, 2), (1100, 200, 1, 1, 4), (1100, 1000, 1, 1, 2),
+                                                 (300, 1200, 20, 0, 4), (40, 30, 600, 0, 4), (1, 64, 4100, 0, 2)])
+def test_oneshot_tiles(gpu, capfd, m, k, ngrp, cplx, tiles):
+    """the tiles of one-shot contractions, as the plan reports them: 4x4
+    fragments where the list they save outweighs the time of one wave's tile,
+    not where few blocks have a long k (or a complex product runs the plan four
+    times); and the product.  Tolerance: an element's k roundings are at most
+    eps |row| |column| each (partial sums included), a random walk of sqrt(k) of
+    them, times 4; |a| |b| bounds the 2-norm of |row| |column| over the elements."""
+    rng = np.random.default_rng(m + k)
+
+    def mats(r, c):
+        return [rng.standard_normal((r, c)) + (1j * rng.standard_normal((r, c)) if cplx else 0) for _ in range(ngrp)]
+
+    A, B = mats(m, k), mats(k, m)
+    lab = [np.arange(ngrp)[:, None]] * 2
+    capfd.readouterr()
+    C = Q.contractQS(Q.QSpace(lab, A, "A", ["x", "y*"]), "2", Q.QSpace(lab, B, "A", ["y", "z*"]), "1", verbose=2)
+    assert f"tiles of up to {tiles} x {tiles} fragments" in capfd.readouterr().err
+    for c, a, b in zip(C.data, A, B):
+        assert np.linalg.norm(c - a @ b) <= 4 * np.sqrt(k) * np.finfo(float).eps * np.linalg.norm(a) * np.linalg.norm(b)
