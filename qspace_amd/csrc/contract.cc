@@ -740,7 +740,10 @@ static std::vector<WorkTarget> plan_targets(const CtrPlan& P) {
 // 64: 345 MFMAs a plan 8.1 / 9.3 / 12.0, 3.2e3 8.8 / 11.6 / 16.3, 5.0e3 9.5 / 11.7
 // / 16.4, 1.0e4 13.1 / 12.9 / 16.8, 1.4e4 14.5 / 13.1 / 17.2.  (Between 24 and 44
 // a SIMD as in stage 1 of H*psi.)  A plan used a few times only (runs > 0) also
-// pays for building its list, 0.03 us an item: up to 4x4 fragments a tile where
+// pays for building its list, 0.03 us an item.  So it takes small tiles only where
+// their items cost less than the at most 4 us an execution that they save (1000
+// blocks of 32 x 32, k = 8: list 0.16 / 0.34 ms with 2x2 / 1x1 tiles, kernel 10 / 12
+// us), and up to 4x4 fragments a tile where
 // that saves more than it adds to the executions.  No wave shares such a tile;
 // the longest takes 0.043 us an MFMA alone, and smaller tiles take that for an
 // average SIMD's MFMAs at least.  List, its upload and the kernel, ms, 2x2 / 4x4
@@ -766,21 +769,31 @@ static void default_policy(CtrPlan& P, int runs) {
   const double mean = mfma / 1024;
   P.policy.wave_max = mean < 8 ? 1 : 2;
   P.policy.group_mfma = mean < 24 ? 8 : mean < 44 ? 32 : 64;
-  if (!runs || frags <= 4096) return;
-  const int mx = P.policy.wave_max;
-  double items = 0, items4 = 0, longest = 0;
-  for (int t = 0; t < P.nT; ++t) {
-    const int mf = (P.M[t] + 15) / 16, nf = (P.N[t] + 15) / 16;
-    if (!mf || !nf) continue;
-    double steps = 0;
-    for (int64_t p = P.pseg[t]; p < P.pseg[t + 1]; ++p) steps += (P.pairs[p].K + 3) / 4;
-    const double tiles = (double)((mf + mx - 1) / mx) * ((nf + mx - 1) / mx);
-    const double mfma = steps * mf * nf / tiles;  // of a tile; a shared one is an item per wave
-    items += mfma > P.policy.group_mfma && steps >= 4 ? 4 * tiles : tiles;
-    items4 += (double)((mf + 3) / 4) * ((nf + 3) / 4);
-    longest = std::max(longest, steps * std::min(mf, 4) * std::min(nf, 4));
+  if (!runs) return;
+  double longest = 0;  // of the 4x4 tiles
+  auto count = [&](int mx, double group) {  // items of the list
+    double items = 0;
+    for (int t = 0; t < P.nT; ++t) {
+      const int mf = (P.M[t] + 15) / 16, nf = (P.N[t] + 15) / 16;
+      if (!mf || !nf) continue;
+      double steps = 0;
+      for (int64_t p = P.pseg[t]; p < P.pseg[t + 1]; ++p) steps += (P.pairs[p].K + 3) / 4;
+      const double tiles = (double)((mf + mx - 1) / mx) * ((nf + mx - 1) / mx);
+      // a tile shared by a workgroup is an item per wave; 4x4 tiles are not
+      items += mx <= 2 && steps * mf * nf / tiles > group && steps >= 4 ? 4 * tiles : tiles;
+      longest = std::max(longest, steps * std::min(mf, 4) * std::min(nf, 4));
+    }
+    return items;
+  };
+  double items = count(P.policy.wave_max, P.policy.group_mfma);
+  const double items2 = count(2, 64);
+  if (kItemUs * (items - items2) > 4.0 * runs) {
+    P.policy.wave_max = 2;
+    P.policy.group_mfma = 64;
+    items = items2;
   }
-  if (kItemUs * (items - items4) > runs * kMfmaUs * std::max(0.0, longest - mean)) P.policy.wave_max = 4;
+  if (frags > 4096 && kItemUs * (items - count(4, 0)) > runs * kMfmaUs * std::max(0.0, longest - mean))
+    P.policy.wave_max = 4;
 }
 
 void plan_upload(CtrPlan& P) {

@@ -615,12 +615,13 @@ def test_split_f32x3_vs_oracle(gpu, heis4000):
 
 @pytest.mark.parametrize("m,k,ngrp,cplx,tiles", [(1000, 64, 1, 0, 2), (1100, 64, 1, 0, 4), (1100, 1000, 1, 0, 4),
                                                  (1100, 3000, 1, 0, 2), (1100, 200, 1, 1, 4), (1100, 1000, 1, 1, 2),
-                                                 (300, 1200, 20, 0, 4), (40, 30, 600, 0, 4), (1, 64, 4100, 0, 2)])
+                                                 (300, 1200, 20, 0, 4), (40, 30, 600, 0, 4), (1, 64, 4100, 0, 2),
+                                                 (32, 8, 40, 0, 1), (32, 8, 1000, 0, 2), (32, 8, 1000, 1, 2)])
 def test_oneshot_tiles(gpu, capfd, m, k, ngrp, cplx, tiles):
     """the tiles of one-shot contractions, as the plan reports them: 4x4
     fragments where the list they save outweighs the time of one wave's tile,
     not where few blocks have a long k (or a complex product runs the plan four
-    times); and the product.  Tolerance: an element's k roundings are at most
+    times), single fragments only where their list is short; and the product.  Tolerance: an element's k roundings are at most
     eps |row| |column| each (partial sums included), a random walk of sqrt(k) of
     them, times 4; |a| |b| bounds the 2-norm of |row| |column| over the elements."""
     rng = np.random.default_rng(m + k)
