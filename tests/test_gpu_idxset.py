@@ -106,7 +106,8 @@ def _labelled(na, nb, nlab, seed, ka=1, kb=1):
 # (records of A, of B, distinct contracted labels): one pair; the sizes of the
 # one-launch engine and one beyond (1024 records, 2048 pairs); many-to-many
 @pytest.mark.parametrize("na,nb,nlab", [(1, 1, 1), (3, 2, 4), (63, 65, 9), (64, 64, 2), (1024, 1024, 512), (1025, 40, 600),
-                                        (40, 1025, 600), (64, 32, 1), (2049, 1, 1), (683, 3, 1), (1024, 1024, 1024)])
+                                        (40, 1025, 600), (64, 32, 1), (2049, 1, 1), (683, 3, 1), (1024, 1024, 1024), (200, 200, 16),
+                                        (1000, 41, 20), (1024, 1024, 511)])
 def test_idxset_engine_sizes(gpu, na, nb, nlab):
     A, B = _labelled(na, nb, nlab, seed=na + 7 * nb)
     _compare(A, [0], B, [0])
