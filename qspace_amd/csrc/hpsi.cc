@@ -91,7 +91,7 @@ struct HpsiPlan {
     int32_t* exps = nullptr;
     SplitLine* dlines = nullptr;
     int nlines = 0;
-    bool lane = false;  // 16 lines per wave (lines adjacent, strided along k)
+    bool lane = false;  // 16 lines per workgroup (lines adjacent, strided along k)
   };
   int nsl = 6;
   SplitSide spHL, spPsi, spT, spHR;
@@ -508,10 +508,11 @@ static void hpsi_autotune(HpsiPlan& H, int reps, double* out) {
 // ---------------------------------------------------------------- split precision
 // Lines of one operand side of a pair list: A side = rows of each A block view
 // (over its K), B side = columns of each B block view.  Blocks shared by
-// several pairs (same offset and strides) share their lines.
+// several pairs (same offset, strides and size: blocks without elements have the
+// offset of the next one) share their lines.
 static std::vector<SplitLine> split_lines(const std::vector<PairDesc>& pairs, const std::vector<WorkTarget>& targets,
                                           bool aside, std::vector<int32_t>& ebase) {
-  std::map<std::tuple<int64_t, int64_t, int64_t, int>, int32_t> seen;
+  std::map<std::tuple<int64_t, int64_t, int64_t, int, int32_t>, int32_t> seen;
   std::vector<SplitLine> lines;
   ebase.assign(pairs.size(), 0);
   for (const WorkTarget& t : targets)
@@ -521,7 +522,7 @@ static std::vector<SplitLine> split_lines(const std::vector<PairDesc>& pairs, co
       const int64_t sl = aside ? ((d.flags & 1) ? d.lda : 1) : ((d.flags & 2) ? 1 : d.ldb);  // between lines
       const int64_t sk = aside ? ((d.flags & 1) ? 1 : d.lda) : ((d.flags & 2) ? d.ldb : 1);  // along a line
       const int n = aside ? t.M : t.N;
-      auto key = std::make_tuple(off, sl, sk, n);
+      auto key = std::make_tuple(off, sl, sk, n, d.K);
       auto it = seen.find(key);
       if (it != seen.end()) {
         ebase[p] = it->second;
@@ -542,8 +543,9 @@ static std::vector<SplitPair> split_pairs(const std::vector<PairDesc>& pairs, co
   for (size_t p = 0; p < pairs.size(); ++p) {
     const PairDesc& d = pairs[p];
     SplitPair& q = v[p];
-    q.pa = la[ea[p]].pbase;
-    q.pb = lb[eb[p]].pbase;
+    // an empty target has no lines (and no items)
+    q.pa = (size_t)ea[p] < la.size() ? la[ea[p]].pbase : 0;
+    q.pb = (size_t)eb[p] < lb.size() ? lb[eb[p]].pbase : 0;
     q.K = d.K;
     q.ea = ea[p];
     q.eb = eb[p];

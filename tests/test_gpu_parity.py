@@ -418,6 +418,29 @@ def test_split_block_sizes(gpu, kw):
         assert np.linalg.norm(got - ref) <= bound * np.linalg.norm(ref), mode
 
 
+@pytest.mark.parametrize("zero", [0, 1, 5, 13])
+def test_split_empty_sector(gpu, zero):
+    """a sector without states on the left bond: its operator blocks have no
+    elements and share their offset (and, with one operator label kept, their
+    row count and strides) with the next block, but not its lines"""
+    HL, psi, HR = gen.heis_hpsi(seed=31, Dstar=40, mu=1.2, sigma=0.4, dmax=6)
+    lab = psi.Q[0][zero, 0]
+
+    def cut(T, legs, wleg):
+        data = [d[tuple(slice(0, 0) if l in legs and T.Q[l][i, 0] == lab else slice(None) for l in range(T.rank))]
+                for i, d in enumerate(T.data)]
+        keep = [i for i in range(len(data)) if wleg is None or T.Q[wleg][i, 0] == 2]
+        return Q.QSpace([q[keep] for q in T.Q], [data[i] for i in keep], T.qtype, T.itags)
+
+    HL, psi, HR = cut(HL, (0, 1), 2), cut(psi, (0,), None), cut(HR, (), 2)
+    x = np.random.RandomState(3).standard_normal(psi.numel())
+    ref = Q.HPsi(HL, psi, HR, hconj=1).apply(x)
+    assert np.linalg.norm(ref) > 0
+    for mode, bound in (("split_bf16", TOL), ("split_f32", 5e-10)):
+        got = Q.HPsi(HL, psi, HR, hconj=1, mode=mode).apply(x)
+        assert np.linalg.norm(got - ref) <= bound * np.linalg.norm(ref), mode
+
+
 def test_split_precision_config4_vs_oracle(gpu, heis4000):
     """config 4 (the headline operator at D* = 4000) in split precision with
     the default slice count: within 1e-12 of the oracle; at full size the
