@@ -59,20 +59,23 @@ __device__ __forceinline__ bool jacobi_cs(double al, double be, double ga, doubl
 
 // rotation of the column pair (ap, aq) of A (m rows) and (vp, vq) of V
 // (n rows) by the 16 lanes of a segment; with R > 0 a lane holds its R
-// elements of each column in registers (m, n <= 16 R), R = 0 runs over the
-// rows in chunks of 4 per lane.  True if the pair was rotated.
-template <int R>
+// elements of each column in registers (8 R < m <= 16 R, or m <= 16 with R = 1;
+// with FULLV n > 8 R too: the first half of the rows needs no mask), R = 0 runs
+// over the rows in chunks of 4 per lane.  True if the pair was rotated.
+template <int R, bool FULLV>
 __device__ __forceinline__ bool rotate_pair(double* ap, double* aq, double* vp, double* vq, int m, int n, int lane,
                                             double tol) {
   constexpr int L = SVD_SEG;
   double c, s;
   if constexpr (R > 0) {
+    auto in_a = [&](int r) { return r < R / 2 || lane + L * r < m; };
+    auto in_v = [&](int r) { return (FULLV && r < R / 2) || lane + L * r < n; };
     double x[R], y[R], u[R], z[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = lane + L * r;
-      x[r] = i < m ? ap[i] : 0.0;
-      y[r] = i < m ? aq[i] : 0.0;
+      x[r] = in_a(r) ? ap[i] : 0.0;
+      y[r] = in_a(r) ? aq[i] : 0.0;
     }
     double al = 0.0, be = 0.0, ga = 0.0;
 #pragma unroll
@@ -88,7 +91,7 @@ __device__ __forceinline__ bool rotate_pair(double* ap, double* aq, double* vp, 
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = lane + L * r;
-      if (i < m) {
+      if (in_a(r)) {
         ap[i] = c * x[r] - s * y[r];
         aq[i] = s * x[r] + c * y[r];
       }
@@ -96,13 +99,13 @@ __device__ __forceinline__ bool rotate_pair(double* ap, double* aq, double* vp, 
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = lane + L * r;
-      u[r] = i < n ? vp[i] : 0.0;
-      z[r] = i < n ? vq[i] : 0.0;
+      u[r] = in_v(r) ? vp[i] : 0.0;
+      z[r] = in_v(r) ? vq[i] : 0.0;
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = lane + L * r;
-      if (i < n) {
+      if (in_v(r)) {
         vp[i] = c * u[r] - s * z[r];
         vq[i] = s * u[r] + c * z[r];
       }
@@ -163,7 +166,7 @@ __device__ __forceinline__ bool rotate_pair(double* ap, double* aq, double* vp, 
 //    w/2 pairs; column w is a dummy when w is odd);
 //  * cross: all pairs (i, np + j), i < np, j < nq: step t pairs i with
 //    (i + t) mod max(np, nq).
-template <int NT, int R, bool CROSS>
+template <int NT, int R, bool CROSS, bool FULLV>
 __device__ __forceinline__ bool jacobi_pairs(double* A, double* V, int np, int nq, int m, int n, double tol,
                                              int* flag) {
   constexpr int L = SVD_SEG;
@@ -195,7 +198,7 @@ __device__ __forceinline__ bool jacobi_pairs(double* A, double* V, int np, int n
         }
         if (p >= w || q >= w) continue;  // the dummy column (whole segment)
       }
-      if (rotate_pair<R>(A + (int64_t)p * m, A + (int64_t)q * m, V + (int64_t)p * n, V + (int64_t)q * n, m, n,
+      if (rotate_pair<R, FULLV>(A + (int64_t)p * m, A + (int64_t)q * m, V + (int64_t)p * n, V + (int64_t)q * n, m, n,
                          lane, tol) &&
           lane == 0)
         *flag = 1;
@@ -207,20 +210,23 @@ __device__ __forceinline__ bool jacobi_pairs(double* A, double* V, int np, int n
   return any;
 }
 
-// the variant for column length m; CROSS: m is longer than SVD_QR_MAX_N
+// the variant for the column lengths: k_jacobi_whole's few columns in registers
+// up to 256 rows, k_jacobi_block's in the registers of its 512 threads for 256 < n
+// <= m <= 512 (without the rows' masks 32 pairs of them spill scalar registers:
+// orthoQS of one 300 x 257 matrix 16.7 / 19.4 ms)
 template <int NT, bool CROSS>
 __device__ __forceinline__ bool jacobi_pairs_m(double* A, double* V, int np, int nq, int m, int n, double tol,
                                                int* flag) {
-  if constexpr (!CROSS) {
-    if (m <= 16) return jacobi_pairs<NT, 1, CROSS>(A, V, np, nq, m, n, tol, flag);
-    if (m <= 32) return jacobi_pairs<NT, 2, CROSS>(A, V, np, nq, m, n, tol, flag);
-    if (m <= 64) return jacobi_pairs<NT, 4, CROSS>(A, V, np, nq, m, n, tol, flag);
-    if (m <= 128) return jacobi_pairs<NT, 8, CROSS>(A, V, np, nq, m, n, tol, flag);
-    if (m <= 256) return jacobi_pairs<NT, 16, CROSS>(A, V, np, nq, m, n, tol, flag);
+  if constexpr (NT == SVD_NT) {
+    if (m <= 16) return jacobi_pairs<NT, 1, CROSS, false>(A, V, np, nq, m, n, tol, flag);
+    if (m <= 32) return jacobi_pairs<NT, 2, CROSS, false>(A, V, np, nq, m, n, tol, flag);
+    if (m <= 64) return jacobi_pairs<NT, 4, CROSS, false>(A, V, np, nq, m, n, tol, flag);
+    if (m <= 128) return jacobi_pairs<NT, 8, CROSS, false>(A, V, np, nq, m, n, tol, flag);
+    if (m <= 256) return jacobi_pairs<NT, 16, CROSS, false>(A, V, np, nq, m, n, tol, flag);
+  } else {
+    if (n > 256 && m <= 512) return jacobi_pairs<NT, 32, CROSS, true>(A, V, np, nq, m, n, tol, flag);
   }
-  if constexpr (NT <= 512)  // registers for 32 elements per lane
-    if (m <= 512) return jacobi_pairs<NT, 32, CROSS>(A, V, np, nq, m, n, tol, flag);
-  return jacobi_pairs<NT, 0, CROSS>(A, V, np, nq, m, n, tol, flag);
+  return jacobi_pairs<NT, 0, CROSS, false>(A, V, np, nq, m, n, tol, flag);
 }
 
 // one-wave workgroups a block is dealt to (gather, scatter): whole columns, or

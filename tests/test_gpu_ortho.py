@@ -171,7 +171,7 @@ def test_ortho_rank_deficient_groups(gpu):
 # m n <= 5120)
 SHAPES = [(1, 1), (2, 2), (5, 2), (16, 16), (17, 16), (40, 17), (33, 32), (96, 96), (97, 97), (130, 96), (128, 97),
           (129, 128), (140, 129), (256, 193), (257, 225), (256, 256), (513, 60), (600, 100), (1024, 33), (1025, 20),
-          (258, 257), (300, 1), (24, 24), (25, 25), (1024, 6), (1024, 7), (640, 8), (641, 8), (213, 24), (214, 24), (2000, 8), (2520, 8), (2521, 8), (1045, 19), (1046, 19), (10111, 1), (12000, 1), (20223, 1)]
+          (258, 257), (512, 257), (513, 258), (300, 1), (24, 24), (25, 25), (1024, 6), (1024, 7), (640, 8), (641, 8), (213, 24), (214, 24), (2000, 8), (2520, 8), (2521, 8), (1045, 19), (1046, 19), (10111, 1), (12000, 1), (20223, 1)]
 
 
 @pytest.mark.parametrize("kind", ["random", "graded", "deficient", "scaled"])
