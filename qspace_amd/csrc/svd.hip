@@ -212,8 +212,8 @@ __device__ __forceinline__ bool jacobi_pairs(double* A, double* V, int np, int n
 
 // the variant for the column lengths: k_jacobi_whole's few columns in registers
 // up to 256 rows, k_jacobi_block's in the registers of its 512 threads for 256 < n
-// <= m <= 512 (without the rows' masks 32 pairs of them spill scalar registers:
-// orthoQS of one 300 x 257 matrix 16.7 / 19.4 ms)
+// <= m <= 512 (masks for all 32 rows of a lane spill scalar registers: orthoQS of
+// one 300 x 257 matrix 19.4 ms, 16.7 with masks for the second half only)
 template <int NT, bool CROSS>
 __device__ __forceinline__ bool jacobi_pairs_m(double* A, double* V, int np, int nq, int m, int n, double tol,
                                                int* flag) {
